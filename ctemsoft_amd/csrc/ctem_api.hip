@@ -1117,6 +1117,131 @@ int32_t expm_depth_mixed(ctem_plan* tp, hipStream_t s, int npad, int nb, float2*
   return CTEM_OK;
 }
 
+// The polynomial of the complex-symmetric form: with squares only, a product needs one operand on chip
+// (ctem_sym.hip). p(B) = s Q3^2 + e1 W2 + e2 B^2 + B with W2 = (B^2 + c B)^2 and Q3 = W2 + d1 B^2 + d2 B
+// matches exp(B) - I through B^7 when c solves c^4 - 10 c^3 + 39 c^2 - 72 c + 60 = 0 (no real root;
+// this one has the smallest coefficients), with 1/s = 20160 c, D = d1 + c^2 = 14 c - 2 c^2,
+// d2 = 84 c - 2 c D, e1 = 1/24 - s (D^2 + 4 c d2), e2 = 1/2 - s d2^2 - e1 c^2; its B^8 coefficient is off by 0.73
+// of 1/8!. theta: see kThetaSym.
+SymCoef sym_coef() {
+  typedef std::complex<double> C;
+  C c(1.5347072799060086, 1.4831613630292302);
+  for (int i = 0; i < 4; i++) {  // to the last bit by Newton's iteration
+    const C p = (((c - 10.0) * c + 39.0) * c - 72.0) * c + 60.0, dp = ((4.0 * c - 30.0) * c + 78.0) * c - 72.0;
+    c -= p / dp;
+  }
+  const C sc = 1.0 / (20160.0 * c), D = 14.0 * c - 2.0 * c * c, d1 = D - c * c, d2 = 84.0 * c - 2.0 * c * D;
+  const C e1 = 1.0 / 24.0 - sc * (D * D + 4.0 * c * d2), e2 = 0.5 - sc * d2 * d2 - e1 * c * c;
+  auto f = [](C v) { return make_float2((float)v.real(), (float)v.imag()); };
+  const float2 zero = make_float2(0.0f, 0.0f), one = make_float2(1.0f, 0.0f);
+  const C bq = e2 - e1 * d1;
+  return SymCoef{{one, one, f(sc)}, {f(c), f(d1), f(e1 / sc)}, {zero, f(d2 - c * d1), f((1.0 - e1 * d2 - c * bq) / sc)},
+                 {zero, zero, f(bq / sc)}};
+}
+// ||B||_1 bound of that polynomial: the truncation adds 2e-8 to the intensities of bcc Fe and fcc Ni (rms
+// over sampled directions in FP64 arithmetic) and 9e-8 on corundum, where degree 8 at theta = 5/4 adds
+// 2e-7, 5e-7 and 4e-9; at 1.07 it would be 1e-6 to 3e-6
+constexpr double kThetaSym = 0.9;
+
+// The complex-symmetric form of expm_depth_split, for the sizes that sym_tiles accepts. Buffers (8 bytes
+// per entry): 0 A as assembled, 1 Q1, 2 Q3 (or the tile images that do not fit on chip), 3 the FP32
+// F for the depth kernel, 4 and 5 the squarings, 6 and 7 E^2 - I and E^4 - I. wmax holds maxima and
+// exponents as in expm_depth_split.
+int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
+                       const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz, int32_t* d_sq,
+                       int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq, int depth_grid,
+                       ChunkSched* cs) {
+  static const SymCoef coef = sym_coef();
+  const int64_t per = (int64_t)npad * npad;
+  auto S = [&](int i) { return (uint16_t*)(W32 + i * per * nb); };
+  auto mx = [&](int i) { return wmax + i * nb; };
+  auto ex = [&](int i) { return (int32_t*)(wmax + (6 + i) * nb); };
+  launch_fill_zero(s, wmax, 12 * sizeof(float) * (size_t)nb);
+  launch_norm_split(s, npad, nb, colpart, amax, kThetaSym, kSmax, d_sq, d_err, ex(0), mx(0));
+  HIPCHK(hipGetLastError());
+  if (cs->known) {
+    h_sq = cs->sq;
+  } else {
+    h_sq.resize(nb);
+    HIPCHK(hipMemcpyAsync(h_sq.data(), d_sq, 4 * (size_t)nb, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+  }
+  int smax = 0;
+  for (int b = 0; b < nb; b++) smax = std::max(smax, h_sq[b]);
+  if (!cs->known) { cs->sq = h_sq; cs->smax = smax; cs->known = true; }
+  launch_sq_check(s, nb, d_sq, smax, d_err);
+  // flops of one symmetric product: the entries on and above the diagonal
+  auto pflops = [&](int b) { return 4.0 * h_n[b] * h_n[b] * (h_n[b] + 1.0); };
+  float2* Ff = W32 + 3 * per * nb;
+  if (sym_onchip(npad)) {
+    double fl = 0.0;
+    for (int b = 0; b < nb; b++) fl += (3 + h_sq[b]) * pflops(b);
+    GemmTimer t{tp, s};
+    t.begin();
+    launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
+    t.end();
+    HIPCHK(hipGetLastError());
+    if (tp) { tp->f_gemm += fl; tp->n_gemm++; }
+    launch_depth(s, npad, nb, nz, Ff, 1, 1, Psi64, spsi, depth_grid);
+    HIPCHK(hipGetLastError());
+    return CTEM_OK;
+  }
+  auto launch = [&](const SymGemm& g, double flops) -> int32_t {
+    GemmTimer t{tp, s};
+    t.begin();
+    launch_sym(s, g);
+    t.end();
+    HIPCHK(hipGetLastError());
+    if (tp) { tp->f_gemm += flops; tp->n_gemm++; }
+    return CTEM_OK;
+  };
+  // matrices past 224 are too large for the on-chip depth kernel: two squarings more give E^2 - I and
+  // E^4 - I (FP32, buffers 6 and 7) for the depth recursion over groups of four depths
+  float2* Ff2 = W32 + 6 * per * nb;
+  float2* Ff4 = W32 + 7 * per * nb;
+  const int extra = 2;
+  double f3 = 0.0;
+  for (int b = 0; b < nb; b++) f3 += pflops(b);
+  auto mk = [&](int c, int x) {
+    SymGemm g{};
+    g.n = npad; g.nb = nb;
+    if (x != 0) g.X = S(x);
+    g.xe = ex(x); g.xmax = mx(x);
+    g.A = W32; g.rs = d_sq; g.bmax = mx(0);
+    g.C = S(c); g.ce = ex(c); g.cmax = mx(c);
+    g.alpha = make_float2(1.0f, 0.0f);
+    return g;
+  };
+  auto finals = [&](SymGemm& g, int at) { g.Cf[0] = Ff; g.Cf[1] = Ff2; g.Cf[2] = Ff4; g.f_sq = d_sq; g.f_at = at; };
+  int32_t rc;
+  const int pc[3] = {1, 2, 5}, px[3] = {0, 1, 2};
+  for (int i = 0; i < 3; i++) {
+    SymGemm g = mk(pc[i], px[i]);
+    g.alpha = coef.alpha[i]; g.bx = coef.bx[i];
+    g.bb = coef.bb[i]; g.has_b = i > 0 ? 1 : 0;
+    if (i == 2) { g.Q = S(1); g.qe = ex(1); g.qmax = mx(1); g.bq = coef.bq[i]; finals(g, 0); }
+    if ((rc = launch(g, f3))) return rc;
+  }
+  const int buf[2] = {5, 4};
+  for (int i = 0; i < smax + extra; i++) {
+    double fl = 0.0;
+    for (int b = 0; b < nb; b++) if (i < h_sq[b] + extra) fl += pflops(b);
+    const int x = buf[i & 1], out = buf[(i + 1) & 1];
+    // the output buffer's maxima were those of two steps back
+    launch_fill_zero(s, mx(out), sizeof(float) * (size_t)nb);
+    SymGemm g = mk(out, x);
+    g.bx = make_float2(2.0f, 0.0f);
+    // every matrix of the chunk in the grid; those whose squarings (plus the extra two) are done
+    // leave at once (counts stay on the device)
+    g.active = d_sq; g.step = i; g.active_add = extra;
+    finals(g, i + 1);
+    if ((rc = launch(g, fl))) return rc;
+  }
+  launch_depth_quad(s, npad, nb, nz, Ff, Ff2, Ff4, Psi64, spsi, depth_grid);
+  HIPCHK(hipGetLastError());
+  return CTEM_OK;
+}
+
 // The mixed form with both stages on CTEM_SPLIT_FP16X3: the same Taylor polynomial and
 // squarings as expm_depth_mixed, with every matrix after the assembly kept in split form
 // (ctem_split.hip), so that the products read their operands without converting them.
@@ -1128,7 +1253,10 @@ int32_t expm_depth_mixed(ctem_plan* tp, hipStream_t s, int npad, int nb, float2*
 int32_t expm_depth_split(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
                          const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz,
                          int32_t* d_sq, int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq,
-                         int depth_grid, bool sym, ChunkSched* cs) {
+                         int depth_grid, bool sym, ChunkSched* cs, bool squares = true) {
+  if (sym && squares && sym_tiles(npad))
+    return expm_depth_sym(tp, s, npad, nb, W32, colpart, amax, wmax, Psi64, spsi, nz, d_sq, d_err, h_n, h_sq, depth_grid,
+                          cs);
   const int64_t per = (int64_t)npad * npad;
   uint16_t* S[6];
   float* mx[6];
@@ -1805,6 +1933,8 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
   const double dzt = p->dz / p->thick;
   const int form = run_form(p, CTEM_PREC_MIXED);
   const bool split = mixed && form == 1;
+  // (its forward keeps the degree-8 polynomial's products: B's gradient is one sum over every direction, as
+  // far from the 64-bit value as its rounding happens to fall, and is not moved by a rounding of another kind)
   const bool sym = split && p->symmetry == 1 && p->cr->centro;
   const size_t budget = (size_t)16 << 30;
   size_t off = 0;
@@ -1864,7 +1994,7 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
                                 c->w.colsum.as<double>(), amax, sym);
           HIPCHK(hipGetLastError());
           rc = expm_depth_split(nullptr, s, npad, nb, W32, c->w.colsum.as<double>(), amax, wmax, c->w.Psi.as<double2>(),
-                                spsi, nz, c->w.sq.as<int32_t>(), p->err.as<int32_t>(), hn, h_sq, c->cu_count, sym, &cs);
+                                spsi, nz, c->w.sq.as<int32_t>(), p->err.as<int32_t>(), hn, h_sq, c->cu_count, sym, &cs, false);
         } else {
           launch_assemble32(s, B, V, R, L, kn, p->cr->mlambda, p->cr->dynupz, p->dz, W32);
           HIPCHK(hipGetLastError());

@@ -186,8 +186,9 @@ CTEM_API int32_t ctem_plan_dynmat(ctem_plan* plan, int32_t ik, double* dynmat, i
  * Ucg and Debye-Waller factors to a measured master pattern. Up to 512 strong beams per
  * direction. */
 CTEM_API int32_t ctem_plan_adjoint(ctem_plan* plan, const double* gdots, double* glut, double* gb);
-/* The same gradient with the mixed forward: psi (and so the intensities the function of gdots was
- * evaluated on) from the plan's mixed form of ctem_plan_run, the backward depth recursion in FP64,
+/* The same gradient with the mixed forward: psi in the mixed form of ctem_plan_run (for an
+ * inversion-symmetric crystal with that form's degree-8 polynomial, within the form's error of
+ * ctem_plan_run's intensities), the backward depth recursion in FP64,
  * and the Frechet derivative of the exponential on split-FP16 products with FP32 accumulation,
  * its squaring stages recomputed. No counterpart in the reference, as ctem_plan_adjoint. Same
  * arguments and limits. */

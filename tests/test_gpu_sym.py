@@ -1,0 +1,52 @@
+"""The complex-symmetric exponential of the mixed form (ctem_sym.hip) at every padded size it has code
+for: one to seven 32 x 32 tiles per side on chip, eight to thirteen through one to three parts per
+product, on bcc Fe and corundum with Bethe cutoffs that give those beam counts. Against the FP64 form, to
+the mixed form's 1e-4 bar, and against the full products (symmetry off), to twice that."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [("fe", w) for w in (4.0, 30.0, 60.0, 100.0, 140.0, 190.0, 250.0, 320.0, 400.0)] + [("al2o3", 280.0), ("al2o3", 400.0)]
+
+
+@pytest.mark.parametrize("crystal,weak", SIZES)
+def test_symmetric_exponential_sizes(crystal, weak):
+    from ctemsoft_amd import ebsd, workloads, xtal
+    wl = workloads.get({"fe": "fe_c1", "al2o3": "al2o3_c2"}[crystal])
+    st, _ = xtal.native_setup(wl.xtal, wl.ekev, wl.dmin, (weak, 2.0 * weak, 0.05))
+    if crystal == "al2o3":  # a LUT box over every difference of two list entries, zero outside the reference's
+        d = st.lut_dim
+        pad = [max(0, int(2 * np.abs(st.hkl[:, a]).max() + st.lut_lo[a])) for a in range(3)]
+        lut = np.pad(st.lut.view(np.complex128).reshape(d[2], d[1], d[0]), [(pad[2],) * 2, (pad[1],) * 2, (pad[0],) * 2])
+        st = ebsd.Setup(st.hkl, st.ucg.view(np.complex128), st.dbdiff, lut, np.asarray(st.lut_lo) - np.array(pad),
+                        st.mlambda, st.dynupz, st.weakcutoff, st.cutoff, st.sgcutoff, st.rmt, st.sites, dsm=st.dsm,
+                        isym=st.isym, usehex=st.usehex)
+    npx, npy = ebsd.lambert_dims(40, st.usehex)
+    ij, k, kn = ebsd.kvectors(npx, npy, st.isym, st.usehex, st.dsm, st.mlambda)
+    ctx = ebsd.Context(0)
+    ctx.upload_crystal(st)
+    lam = np.exp(-np.arange(1, 11) / 8.0).astype(np.float32)
+    probe = ctx.plan(k, kn, lam, 1.0, 10.0)
+    ns, _ = probe.select()
+    probe.close()
+    pad = np.maximum(32, (ns + 31) // 32 * 32)
+    # of each padded size: the smallest, the largest and a few more
+    pick = np.unique(np.concatenate([np.concatenate([i[np.argsort(ns[i], kind="stable")][[0, -1]], i[:4]])
+                                     for i in (np.flatnonzero(pad == p) for p in np.unique(pad))]))
+    plan = ctx.plan(k[pick], kn[pick], lam, 1.0, 10.0)
+    plan.run("fp64")
+    ref = plan.dots().copy()
+    assert plan.set_symmetry(1)
+    plan.run("mixed")
+    got = plan.dots().copy()
+    assert not plan.set_symmetry(0)
+    plan.run("mixed")
+    full = plan.dots().copy()
+    plan.close()
+    ctx.close()
+    rel = (np.abs(got - ref) / np.abs(ref)).max(1)
+    for p in np.unique(pad[pick]):
+        print(f"{crystal} {weak}: npad {p}: {rel[pad[pick] == p].max():.1e}", flush=True)
+    assert np.isfinite(got).all() and rel.max() < 1e-4
+    assert (np.abs(got - full) / np.abs(ref)).max() < 2e-4
