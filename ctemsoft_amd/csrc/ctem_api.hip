@@ -2545,6 +2545,7 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
   // 5 x 2 matrices of their exponentials
   auto per_dir = [&](int npad) -> size_t {
     const size_t per = (size_t)npad * npad;
+    if (ecp_small(npad)) return per * sizeof(double2) + 64;  // A only
     if (bloch) return (per + 8 * per + 40 * per) * sizeof(double2) + 64;
     const size_t nzp = (size_t)(numt + 31) / 32 * 32;
     return (6 * per + (size_t)npad * numt) * sizeof(double2) + (size_t)(npad / 32) * nzp * 8 + 64;
@@ -2554,7 +2555,9 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
     const int npad = kv.first, nbk = (int)kv.second.size();
     const size_t per = (size_t)npad * npad;
     const size_t nb = (size_t)std::max(1, (int)std::min<size_t>(nbk, std::max<size_t>(1, chunk_budget(p) / per_dir(npad))));
-    if (bloch) {
+    if (ecp_small(npad)) {
+      a = std::max(a, per * nb * sizeof(double2));
+    } else if (bloch) {
       a = std::max(a, 8 * per * nb * sizeof(double2));
       w = std::max(w, 40 * per * nb * sizeof(double2));
       ps = std::max(ps, per * nb * sizeof(double2));
@@ -2596,7 +2599,19 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
       Bucket B{npad, nb, p->dirs.as<int32_t>() + off + c0};
       std::vector<int> hn;
       std::vector<int32_t> hsq;
-      if (!bloch) {
+      if (ecp_small(npad)) {
+        double2* A = c->w.A.as<double2>();
+        if (bloch) {
+          launch_assemble(s, B, V, R, L, p->kn.as<double>(), p->cr->mlambda, p->cr->dynupz, 1.0, A);
+          launch_ecp_bloch_small(s, B, V, R, LE, A, (double)p->ecp_t0, (double)p->ecp_dt, nt, p->ecp_thick.as<float>(),
+                                 p->ecp_nat, p->numk, p->err.as<int32_t>(), p->ecp_sr.as<float>());
+        } else {
+          launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, A);
+          launch_ecp_scat_small(s, B, V, R, LE, A, numt, p->ecp_store.as<int32_t>(), p->ecp_nat, p->numk,
+                                p->err.as<int32_t>(), p->ecp_sr.as<float>());
+        }
+        HIPCHK(hipGetLastError());
+      } else if (!bloch) {
         for (int b = 0; b < nb; b++) hn.push_back(p->h_nns[kv.second[c0 + b]]);
         // Minp = DynMat * dcmplx(0, cPi mLambda), Azz = MatrixExponential(Minp, zintstep, 'Pade')
         launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, c->w.A.as<double2>());
