@@ -815,10 +815,11 @@ constexpr int kSmax = 48;
 // receives the squaring counts.
 // cs (may be null): with cs->known the squaring counts of this chunk are taken from it and not
 // read back (no host synchronisation); otherwise they are read back and stored in it.
+// own: the matrices' sizes where the rest of each is zero (absent: npad).
 double2* expm_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, double2* W,
                    int32_t* d_sq, int32_t* d_err, const std::vector<int>& h_n,
                    std::vector<int32_t>& h_sq, int32_t& rc_out, double* d_amod = nullptr,
-                   std::vector<double>* h_amod = nullptr, ChunkSched* cs = nullptr) {
+                   std::vector<double>* h_amod = nullptr, ChunkSched* cs = nullptr, MatSizes own = {}) {
   rc_out = CTEM_OK;
   const int64_t per = (int64_t)npad * npad;
   double2* A2 = W;
@@ -849,7 +850,8 @@ double2* expm_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, d
 
   auto sq_gemm = [&](double2* C, const double2* X, const double2* Y, double betaI,
                      std::initializer_list<std::pair<const double2*, double>> ms,
-                     const int32_t* active, int step, double flops) -> int32_t {
+                     const int32_t* active, int step, double flops, double2* C2 = nullptr,
+                     double betaI2 = 0.0) -> int32_t {
     ZGemm g{};
     g.m = npad; g.n = npad; g.k = npad;
     g.ldx = g.ldy = g.ldc = g.ldm = npad;
@@ -858,6 +860,7 @@ double2* expm_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, d
     int q = 0;
     for (auto& m : ms) { g.M[q] = m.first; g.beta[q] = m.second; q++; }
     g.active = active; g.step = step; g.nb = nb;
+    g.own = own; g.trim = 7; g.C2 = C2; g.betaI2 = betaI2;
     GemmTimer t{tp, s};
     t.begin();
     launch_zgemm(s, g);
@@ -870,13 +873,9 @@ double2* expm_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, d
   const double f3 = 8.0 * n3;
   if ((rc = sq_gemm(A2, A, A, 0.0, {}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
   if ((rc = sq_gemm(A3, A, A2, 0.0, {}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
-  if ((rc = sq_gemm(A4, A2, A2, 0.0, {}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
-  {
-    const double2* M[4] = {A, A2, A3, A4};
-    const double beta[4] = {inv_fact(13), inv_fact(14), inv_fact(15), inv_fact(16)};
-    launch_combo(s, npad, nb, H, inv_fact(12), M, beta);
-    EXPM_CHK(hipGetLastError());
-  }
+  // A4, and H = I / 12! + A / 13! + A2 / 14! + A3 / 15! + A4 / 16! from the same product
+  if ((rc = sq_gemm(A4, A2, A2, 0.0, {{A, inv_fact(13)}, {A2, inv_fact(14)}, {A3, inv_fact(15)}, {nullptr, inv_fact(16)}},
+                    nullptr, 0, f3, H, inv_fact(12)))) { rc_out = rc; return nullptr; }
   if ((rc = sq_gemm(T, A4, H, inv_fact(8), {{A, inv_fact(9)}, {A2, inv_fact(10)}, {A3, inv_fact(11)}}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
   if ((rc = sq_gemm(H, A4, T, inv_fact(4), {{A, inv_fact(5)}, {A2, inv_fact(6)}, {A3, inv_fact(7)}}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
   if ((rc = sq_gemm(T, A4, H, 1.0, {{A, 1.0}, {A2, inv_fact(2)}, {A3, inv_fact(3)}}, nullptr, 0, f3))) { rc_out = rc; return nullptr; }
@@ -895,12 +894,12 @@ double2* expm_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, d
 
 // expm of the block matrix [[X, Y], [0, X]] held as the pair (X, Y) (npad x npad each): the same
 // degree-16 Taylor evaluation and squarings as expm_fp64, every product of two pairs
-// (X1 X2, X1 Y2 + Y1 X2) taken as three n-size GEMMs (the dense 2n-size product is eight). X and
+// (X1 X2, X1 Y2 + Y1 X2) taken as three n-size GEMMs in one launch (the dense 2n-size product is eight). X and
 // Y are scaled in place; W holds 10 nb npad^2 entries. Returns the pair (E, L) in W: E at the
 // returned pointer, L at E + 5 nb npad^2 (L = the Frechet derivative of expm at X in the direction
 // Y when X, Y are unscaled on entry).
 double2* expm_pair_fp64(hipStream_t s, int npad, int nb, double2* X, double2* Y, double2* W, int32_t* d_sq,
-                        int32_t* d_err, std::vector<int32_t>& h_sq, int32_t& rc_out) {
+                        int32_t* d_err, std::vector<int32_t>& h_sq, int32_t& rc_out, MatSizes own) {
   rc_out = CTEM_OK;
   const int64_t per = (int64_t)npad * npad;
   const int64_t half = 5 * per * nb;  // X parts in W[0, half), Y parts in W[half, 2 half)
@@ -922,32 +921,26 @@ double2* expm_pair_fp64(hipStream_t s, int npad, int nb, double2* X, double2* Y,
   PAIR_CHK(hipStreamSynchronize(s));
   int smax = 0;
   for (int b = 0; b < nb; b++) smax = std::max(smax, h_sq[b]);
-  // C = X*Y + betaI I + sum beta_j M_j over the nb matrices (M may be C itself: the epilogue reads
-  // each addend element before it writes that element of C)
-  auto gemm = [&](double2* C, const double2* A_, const double2* B_, double betaI,
-                  std::initializer_list<std::pair<const double2*, double>> ms, const int32_t* active,
-                  int step) -> bool {
+  // (CX, CY) = (AX, AY)(BX, BY) + betaI (I, 0) + sum beta_j (MX_j, MY_j)
+  auto pmul = [&](double2* CX, double2* CY, const double2* AX, const double2* AY, const double2* BX,
+                  const double2* BY, double betaI, std::initializer_list<std::pair<const double2*, double>> mx,
+                  std::initializer_list<const double2*> my, const int32_t* active, int step) -> bool {
     ZGemm g{};
     g.m = g.n = g.k = npad;
     g.ldx = g.ldy = g.ldc = g.ldm = npad;
-    g.X = A_; g.sx = per; g.Y = B_; g.sy = per; g.C = C; g.sc = per; g.sm = per;
+    g.X = AX; g.sx = per; g.Y = BX; g.sy = per; g.C = CX; g.sc = per; g.sm = per;
+    g.Xd = AY; g.Yd = BY; g.Cd = CY;
     g.alpha = 1.0; g.betaI = betaI;
     int q = 0;
-    for (auto& m : ms) { g.M[q] = m.first; g.beta[q] = m.second; q++; }
+    for (auto& m : mx) { g.M[q] = m.first; g.beta[q] = m.second; q++; }
+    q = 0;
+    for (auto m : my) g.Md[q++] = m;
     g.active = active; g.step = step; g.nb = nb;
+    g.own = own; g.trim = 7;
     launch_zgemm(s, g);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { rc_out = fail(CTEM_E_HIP, "pair product: %s", hipGetErrorString(e)); return false; }
     return true;
-  };
-  // (CX, CY) = (AX, AY)(BX, BY) + betaI (I, 0) + sum beta_j (MX_j, MY_j)
-  auto pmul = [&](double2* CX, double2* CY, const double2* AX, const double2* AY, const double2* BX,
-                  const double2* BY, double betaI, std::initializer_list<std::pair<const double2*, double>> mx,
-                  std::initializer_list<std::pair<const double2*, double>> my, const int32_t* active,
-                  int step) -> bool {
-    if (!gemm(CX, AX, BX, betaI, mx, active, step)) return false;
-    if (!gemm(CY, AX, BY, 0.0, my, active, step)) return false;
-    return gemm(CY, AY, BX, 0.0, {{CY, 1.0}}, active, step);
   };
   if (!pmul(X2, Y2, X, Y, X, Y, 0.0, {}, {}, nullptr, 0)) return nullptr;
   if (!pmul(X3, Y3, X, Y, X2, Y2, 0.0, {}, {}, nullptr, 0)) return nullptr;
@@ -961,13 +954,13 @@ double2* expm_pair_fp64(hipStream_t s, int npad, int nb, double2* X, double2* Y,
     PAIR_CHK(hipGetLastError());
   }
   if (!pmul(XT, YT, X4, Y4, XH, YH, inv_fact(8), {{X, inv_fact(9)}, {X2, inv_fact(10)}, {X3, inv_fact(11)}},
-            {{Y, inv_fact(9)}, {Y2, inv_fact(10)}, {Y3, inv_fact(11)}}, nullptr, 0))
+            {Y, Y2, Y3}, nullptr, 0))
     return nullptr;
   if (!pmul(XH, YH, X4, Y4, XT, YT, inv_fact(4), {{X, inv_fact(5)}, {X2, inv_fact(6)}, {X3, inv_fact(7)}},
-            {{Y, inv_fact(5)}, {Y2, inv_fact(6)}, {Y3, inv_fact(7)}}, nullptr, 0))
+            {Y, Y2, Y3}, nullptr, 0))
     return nullptr;
   if (!pmul(XT, YT, X4, Y4, XH, YH, 1.0, {{X, 1.0}, {X2, inv_fact(2)}, {X3, inv_fact(3)}},
-            {{Y, 1.0}, {Y2, inv_fact(2)}, {Y3, inv_fact(3)}}, nullptr, 0))
+            {Y, Y2, Y3}, nullptr, 0))
     return nullptr;
   double2* bx[2] = {XT, XH};
   double2* by[2] = {YT, YH};
@@ -986,9 +979,9 @@ int32_t expm_depth_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2*
                         double2* Psi, int64_t spsi, int nz, int32_t* d_sq, int32_t* d_err,
                         const std::vector<int>& h_n, std::vector<int32_t>& h_sq, int depth_grid,
                         double* d_amod = nullptr, std::vector<double>* h_amod = nullptr,
-                        ChunkSched* cs = nullptr) {
+                        ChunkSched* cs = nullptr, MatSizes own = {}) {
   int32_t rc;
-  double2* E = expm_fp64(tp, s, npad, nb, A, W, d_sq, d_err, h_n, h_sq, rc, d_amod, h_amod, cs);
+  double2* E = expm_fp64(tp, s, npad, nb, A, W, d_sq, d_err, h_n, h_sq, rc, d_amod, h_amod, cs, own);
   if (!E) return rc;
   launch_depth(s, npad, nb, nz, E, 0, 0, Psi, spsi, depth_grid);
   HIPCHK(hipGetLastError());
@@ -1598,7 +1591,7 @@ int32_t run_enqueue(ctem_plan* p, int32_t precision, bool timed, bool sync_ok, d
         std::vector<double> hmod;
         rc = expm_depth_fp64(tp, s, npad, nb, c->w.A.as<double2>(), c->w.W.as<double2>(), c->w.Psi.as<double2>(), spsi,
                              p->nz, c->w.sq.as<int32_t>(), p->err.as<int32_t>(), hn, p->h_sq, c->cu_count,
-                             c->w.amod.as<double>(), &hmod, &cs);
+                             c->w.amod.as<double>(), &hmod, &cs, MatSizes{V.nns, B.dirs});
         if (!rc && first && fa) {
           for (int b = 0; b < nb; b++) {
             const int d = kv.second[c0 + b];
@@ -2010,7 +2003,7 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
         launch_assemble(s, B, V, R, L, kn, p->cr->mlambda, p->cr->dynupz, p->dz, A);
         HIPCHK(hipGetLastError());
         E = expm_fp64(nullptr, s, npad, nb, A, c->w.W.as<double2>(), c->w.sq.as<int32_t>(), p->err.as<int32_t>(), hn,
-                      h_sq, rc);
+                      h_sq, rc, nullptr, nullptr, nullptr, MatSizes{V.nns, B.dirs});
         if (!E) return rc;
         launch_depth(s, npad, nb, nz, E, 0, 0, c->w.Psi.as<double2>(), spsi, c->cu_count);
       }
@@ -2030,6 +2023,7 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
         g.Y = c->w.Psi.as<double2>(); g.sy = spsi;
         g.C = c->w.aQ.as<double2>(); g.sc = spsi;
         g.alpha = 1.0; g.nb = nb;
+        g.own = MatSizes{V.nns, B.dirs}; g.trim = 1 | 4;
         launch_zgemm(s, g);
         HIPCHK(hipGetLastError());
       }
@@ -2045,6 +2039,7 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
         g.Y = c->w.aHm.as<double2>(); g.sy = spsi;
         g.C = c->w.aEbar.as<double2>(); g.sc = per;
         g.alpha = 1.0; g.nb = nb;
+        g.own = MatSizes{V.nns, B.dirs}; g.trim = 1 | 2;
         launch_zgemm(s, g);
         HIPCHK(hipGetLastError());
       }
@@ -2070,7 +2065,7 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
         launch_adj_pair(s, npad, nb, A, c->w.aEbar.as<double2>(), c->w.aSig.as<double>(), PX, PY);
         HIPCHK(hipGetLastError());
         double2* T2 = expm_pair_fp64(s, npad, nb, PX, PY, c->w.aW2.as<double2>(), c->w.sq.as<int32_t>(),
-                                     p->err.as<int32_t>(), h_sq2, rc);
+                                     p->err.as<int32_t>(), h_sq2, rc, MatSizes{V.nns, B.dirs});
         if (!T2) return rc;
         launch_adj_extract(s, B, V, kn, p->dz, T2 + 5 * per * nb, npad, c->w.aSig.as<double>(),
                            c->w.aDbar.as<double2>());
@@ -2264,7 +2259,8 @@ extern "C" int32_t ctem_calclgh3_static(ctem_ctx* c, const double* dmat, double*
   HIPCHK(hipGetLastError());
   std::vector<int> hn{nn};
   std::vector<int32_t> hsq;
-  int32_t rc = expm_depth_fp64(nullptr, s, npad, 1, A, W, Psi, spsi, izz, d_sq, d_err, hn, hsq, c->cu_count);
+  int32_t rc = expm_depth_fp64(nullptr, s, npad, 1, A, W, Psi, spsi, izz, d_sq, d_err, hn, hsq, c->cu_count,
+                               nullptr, nullptr, nullptr, MatSizes{nullptr, nullptr, nn});
   if (rc) return rc;
   const int32_t nnv[2] = {nn, 0};
   HIPCHK(hipMemcpyAsync(d_nns, nnv, 8, hipMemcpyHostToDevice, s));
@@ -2322,7 +2318,8 @@ extern "C" int32_t ctem_calclgh3(ctem_ctx* c, const double* dmat, double* lgh, d
   std::vector<int> hn{nn};
   std::vector<int32_t> hsq;
   rc = expm_depth_fp64(nullptr, s, npad, 1, c->s_A.as<double2>(), c->s_W.as<double2>(), c->s_Psi.as<double2>(),
-                       spsi, izz, c->s_sq.as<int32_t>(), c->s_err.as<int32_t>(), hn, hsq, c->cu_count);
+                       spsi, izz, c->s_sq.as<int32_t>(), c->s_err.as<int32_t>(), hn, hsq, c->cu_count, nullptr, nullptr,
+                       nullptr, MatSizes{nullptr, nullptr, nn});
   if (rc) return rc;
   // Lgh through the contraction kernel with no sites: a one-entry plan view
   const int32_t zero4[4] = {0, 0, 0, 0};

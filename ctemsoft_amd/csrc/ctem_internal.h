@@ -185,6 +185,13 @@ void launch_dynmat(hipStream_t s, const Bucket& B, const BeamView& V, const DevR
 void launch_norm_scale(hipStream_t s, int32_t npad, int32_t nb, double2* A, double theta,
                        int32_t smax, int32_t* sq, int32_t* err, double* amod);
 
+// the own sizes of padded matrices: nns[dirs[b]], or n for all
+struct MatSizes {
+  const int32_t* nns = nullptr;
+  const int32_t* dirs = nullptr;
+  int32_t n = 0;
+};
+
 // Batched complex GEMM C = alpha*X*Y + betaI*I + sum_j beta_j*M_j on FP64 MFMA.
 struct ZGemm {
   int32_t m, n, k;       // C is m x n, X is m x k, Y is k x n (column-major)
@@ -197,6 +204,14 @@ struct ZGemm {
   const double2* M[4]; double beta[4]; int64_t sm;
   const int32_t* active; int32_t step;   // skip matrix b when step >= active[b]
   int32_t nb;
+  // The matrices' own sizes (all absent: the full ones); trim says which of m (1), n (2), k (4) they cut. X's
+  // columns and Y's rows past them are zero off the diagonal, and C there receives the other terms
+  MatSizes own; int32_t trim;
+  // with C2 the addends go to it instead of to C: C2 = betaI2 I + sum_j<3 beta_j M_j + beta_3 C
+  double2* C2; double betaI2;
+  // with Xd a second result from the same launch, of the pair product (X, Xd)(Y, Yd):
+  // Cd = alpha (X Yd + Xd Y) + sum_j beta_j Md_j
+  const double2* Xd; const double2* Yd; double2* Cd; const double2* Md[4];
 };
 void launch_zgemm(hipStream_t s, const ZGemm& g);
 

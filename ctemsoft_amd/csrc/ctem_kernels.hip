@@ -347,104 +347,274 @@ void launch_norm_scale(hipStream_t s, int32_t npad, int32_t nb, double2* A, doub
 }
 
 // ------------------------------------------------------------------------------------------
-// batched complex GEMM, FP64 MFMA. Workgroup tile 64x64, 4 waves of 32x32, K chunks of 16
-// staged through LDS. MFMA 16x16x4 f64 operand layout (lane l): A[l%16][l/16],
-// B[l/16][l%16]; result element e of lane l is C[l/16 + 4*e][l%16] (rows interleaved by 4,
-// unlike the f32/bf16 16x16 variants whose lane holds four consecutive rows).
-#define ZG_LDS 65
-__global__ __launch_bounds__(256) void k_zgemm(ZGemm g) {
-  const int tm = (g.m + 63) / 64, tn = (g.n + 63) / 64;
-  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int b = lb / (tm * tn);
-  const int t = lb % (tm * tn);
-  const int bm = (t % tm) * 64, bn = (t / tm) * 64;
-  if (g.active && g.step >= g.active[b]) return;
-  const double2* X = g.X + (int64_t)b * g.sx;
-  const double2* Y = g.Y + (int64_t)b * g.sy;
-  double2* C = g.C + (int64_t)b * g.sc;
-
-  __shared__ double As_r[16][ZG_LDS], As_i[16][ZG_LDS], Bs_r[16][ZG_LDS], Bs_i[16][ZG_LDS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const int l16 = lane & 15, l4 = lane >> 4;
-  // waves whose 32x32 sub-tile lies wholly in the padding only help to stage operands
-  const bool wave_live = (bm + wm < g.m) && (bn + wn < g.n);
-
-  double4v cr[2][2], ci[2][2];
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) { cr[i][j] = (double4v){0, 0, 0, 0}; ci[i][j] = (double4v){0, 0, 0, 0}; }
-
-  // register-prefetch pipeline: the global loads of chunk k0+16 are in flight while the
-  // MFMAs of chunk k0 run from LDS
-  double2 ra[4], rb[4];
-  auto gload = [&](int k0) {
-    for (int r = 0; r < 4; r++) {
-      const int mm = tid & 63, kk = (tid >> 6) + 4 * r;
-      const int row = bm + mm, col = k0 + kk;
-      ra[r] = (row < g.m && col < g.k) ? X[(int64_t)col * g.ldx + row] : make_double2(0.0, 0.0);
-    }
-    for (int r = 0; r < 4; r++) {
-      const int kk = tid & 15, nn = (tid >> 4) + 16 * r;
-      const int row = k0 + kk, col = bn + nn;
-      rb[r] = (row < g.k && col < g.n) ? Y[(int64_t)col * g.ldy + row] : make_double2(0.0, 0.0);
-    }
-  };
-  gload(0);
-  for (int k0 = 0; k0 < g.k; k0 += 16) {
-    __syncthreads();
-    for (int r = 0; r < 4; r++) {
-      const int mm = tid & 63, kk = (tid >> 6) + 4 * r;
-      As_r[kk][mm] = ra[r].x;
-      As_i[kk][mm] = ra[r].y;
-      const int kb = tid & 15, nn = (tid >> 4) + 16 * r;
-      Bs_r[kb][nn] = rb[r].x;
-      Bs_i[kb][nn] = rb[r].y;
-    }
-    __syncthreads();
-    if (k0 + 16 < g.k) gload(k0 + 16);
-    if (!wave_live) continue;
+// batched complex GEMM, FP64 MFMA 16x16x4 (lane l: A[l%16][l/16], B[l/16][l%16]; result element e of
+// lane l is C[l/16 + 4*e][l%16], rows interleaved by 4 unlike the f32/bf16 16x16 variants whose lane holds
+// four consecutive rows). Y is passed as A and X as B, so that 16 lanes hold 16 consecutive rows of C.
+//
+// k_zgemm: workgroup tile 64x64, 4 waves of 32x32, K in chunks of 8 that the load unit writes to LDS (two
+// buffers, one barrier a chunk). Bound by the matrix cores: 64 MFMAs of 64 cycles per SIMD and chunk
+// against 16 KB staged. A matrix's own size n (its beams, of npad) cuts K to multiples of 8 and the waves'
+// tiles to multiples of 16; the zero padding past it is written, not multiplied. The waves' places in the
+// tile turn with the matrix, so that the waves with cut tiles are spread over the four SIMDs. 110 registers,
+// four workgroups per CU (three are 15% slower). Measured on one MI355X against chunks staged through registers
+// with the accumulators moved each chunk: the products of 1,326 matrices of 87-115 beams and their adjoint
+// pairs 26.0 -> 16.8 ms, half of it matrix-core time, with 40 GB of operands moved; bcc Fe FP64 master of
+// up to 224 beams 34.4 -> 26 ms.
+constexpr int kZgemmFew = 256;  // 64x64 tiles: one per CU
+struct ZgOperands {  // of one result: np products of X[p] and Y[p]
+  const double2* X[2];
+  const double2* Y[2];
+  const double2* M[4];
+  double2* C;
+  double betaI;
+  int np;
+};
+__device__ __forceinline__ ZgOperands zg_operands(const ZGemm& g, bool dual) {
+  ZgOperands o;
+  o.X[0] = g.X; o.X[1] = g.Xd;
+  o.Y[0] = dual ? g.Yd : g.Y; o.Y[1] = g.Y;
 #pragma unroll
-    for (int ks = 0; ks < 16; ks += 4) {
-      double a_r[2], a_i[2], b_r[2], b_i[2];
-      for (int i = 0; i < 2; i++) {
-        a_r[i] = As_r[ks + l4][wm + 16 * i + l16];
-        a_i[i] = As_i[ks + l4][wm + 16 * i + l16];
-        b_r[i] = Bs_r[ks + l4][wn + 16 * i + l16];
-        b_i[i] = Bs_i[ks + l4][wn + 16 * i + l16];
+  for (int q = 0; q < 4; q++) o.M[q] = dual ? g.Md[q] : g.M[q];
+  o.C = dual ? g.Cd : g.C;
+  o.betaI = dual ? 0.0 : g.betaI;
+  o.np = dual ? 2 : 1;
+  return o;
+}
+
+struct ZgTile {
+  ZgOperands o;
+  int bm, bn, wm, wn, me, ne, ke;
+};
+
+// 1 KB from global memory (16 bytes at base + off of each lane) to LDS (dst + 16 lane), asynchronously;
+// waited for by s_waitcnt vmcnt(0) before the barrier ahead of the first read
+__device__ __forceinline__ void zg_to_lds(const double2* base, unsigned off, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(dst), "v"(off), "s"(base) : "memory", "m0");
+}
+
+template <int NI, int NJ>
+__device__ __forceinline__ void zg_run(const ZGemm& g, const ZgTile& t, int b, int wave, int lane, double2* lds) {
+  const ZgOperands& o = t.o;
+  double2* C = o.C + (int64_t)b * g.sc;
+  const int l16 = lane & 15, l4 = lane >> 4;
+  double4v cr[2][2], ci[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) { cr[i][j] = (double4v){0, 0, 0, 0}; ci[i][j] = (double4v){0, 0, 0, 0}; }
+  // LDS, per buffer: X [8 k][64 rows], then Y [64 columns][8 k] with column c's k at place k ^ ((c >> 1) & 7),
+  // so that the 16 columns of a read cover all banks
+  constexpr int kBuf = 1024;
+  const unsigned l0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+  const int nk1 = (t.bm < t.me && t.bn < t.ne) ? (t.ke + 7) >> 3 : 0, nk = nk1 * o.np;
+  // (nothing past the last cut tile is read)
+  const int mx = min(g.m, (t.me + 15) & ~15) - 1, nx = min(g.n, (t.ne + 15) & ~15) - 1;
+  const unsigned xoff = 16u * (unsigned)min(t.bm + lane, mx);
+  unsigned ycol[2];
+  int yk[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int nn = (wave * 2 + h) * 8 + (lane >> 3);
+    ycol[h] = (unsigned)min(t.bn + nn, nx) * (unsigned)g.ldy;
+    yk[h] = (lane & 7) ^ ((nn >> 1) & 7);
+  }
+  auto issue = [&](int cc, int z) {
+    const int second = cc >= nk1, c = second ? cc - nk1 : cc;
+    const double2* X = o.X[second] + (int64_t)b * g.sx;
+    const double2* Y = o.Y[second] + (int64_t)b * g.sy;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int kk = wave * 2 + h, k = min(8 * c + kk, g.k - 1);
+      zg_to_lds(X + (int64_t)k * g.ldx, xoff, l0 + 16 * (z * kBuf + kk * 64));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      zg_to_lds(Y + 8 * c, 16u * (ycol[h] + (unsigned)min(yk[h], g.k - 1 - 8 * c)),
+                l0 + 16 * (z * kBuf + 512 + (wave * 2 + h) * 64));
+  };
+  if (nk) issue(0, 0);
+  for (int c = 0; c < nk; c++) {
+    const int z = c & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // chunk c has arrived, and every wave is done with the other buffer
+    asm volatile("" ::: "memory");
+    if (c + 1 < nk) issue(c + 1, z ^ 1);
+    const int kc = 8 * (c >= nk1 ? c - nk1 : c);
+    if (kc + 8 > g.k) {  // the end of a K that isn't a multiple of 8
+      const int rem = g.k - kc;
+      for (int q = wave * 64 + lane; q < 64 * 8; q += 256) {
+        if (q >> 6 >= rem) lds[z * kBuf + q] = make_double2(0.0, 0.0);
+        if (((q & 7) ^ ((q >> 4) & 7)) >= rem) lds[z * kBuf + 512 + q] = make_double2(0.0, 0.0);
       }
-      for (int i = 0; i < 2; i++)
-        for (int j = 0; j < 2; j++) {
-          cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a_r[i], b_r[j], cr[i][j], 0, 0, 0);
-          ci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a_r[i], b_i[j], ci[i][j], 0, 0, 0);
-          cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a_i[i], b_i[j], cr[i][j], 0, 0, 0);
-          ci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a_i[i], b_r[j], ci[i][j], 0, 0, 0);
+      __syncthreads();
+    }
+    const double2* xs = lds + z * kBuf + t.wm + l16;
+    const double2* ys = lds + z * kBuf + 512 + (t.wn + l16) * 8;
+#pragma unroll
+    for (int ks = 0; ks < 8; ks += 4) {
+      double2 x[2], y[2];
+#pragma unroll
+      for (int i = 0; i < NI; i++) x[i] = xs[(ks + l4) * 64 + 16 * i];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) y[j] = ys[128 * j + ((ks + l4) ^ (l16 >> 1))];
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+          cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[j].x, x[i].x, cr[i][j], 0, 0, 0);
+          ci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[j].y, x[i].x, ci[i][j], 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+          cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[j].y, -x[i].y, cr[i][j], 0, 0, 0);
+          ci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[j].x, x[i].y, ci[i][j], 0, 0, 0);
         }
     }
   }
-  if (!wave_live) return;
   // epilogue
+  const int r0 = t.bm + t.wm + l16, c0 = t.bn + t.wn + l4;
+#pragma unroll
   for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int row = r0 + 16 * i;
+      double2 v[4], u[4];
+#pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int row = bm + wm + 16 * i + l4 + 4 * e;
-        const int col = bn + wn + 16 * j + l16;
-        if (row < g.m && col < g.n) {
-          double vr = g.alpha * cr[i][j][e], vi = g.alpha * ci[i][j][e];
-          if (row == col) vr += g.betaI;
-          for (int q = 0; q < 4; q++)
-            if (g.M[q]) {
-              const double2 mv = g.M[q][(int64_t)b * g.sm + (int64_t)col * g.ldm + row];
-              vr += g.beta[q] * mv.x;
-              vi += g.beta[q] * mv.y;
-            }
-          C[(int64_t)col * g.ldc + row] = make_double2(vr, vi);
+        v[e] = make_double2(g.alpha * cr[i][j][e], g.alpha * ci[i][j][e]);
+        const bool diag = row == c0 + 16 * j + 4 * e;
+        if (diag) v[e].x += o.betaI;
+        if (g.C2) {
+          u[e] = v[e];
+          v[e] = make_double2(diag ? g.betaI2 : 0.0, 0.0);
         }
       }
+      if (row >= g.m) continue;
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (o.M[q]) {
+          const double2* M = o.M[q] + (int64_t)b * g.sm + row;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int col = c0 + 16 * j + 4 * e;
+            const double2 mv = col < g.n ? M[(int64_t)col * g.ldm] : make_double2(0.0, 0.0);
+            v[e].x += g.beta[q] * mv.x;
+            v[e].y += g.beta[q] * mv.y;
+          }
+        }
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int col = c0 + 16 * j + 4 * e;
+        if (col >= g.n) continue;
+        const int64_t at = (int64_t)col * g.ldc + row;
+        if (g.C2) {
+          C[at] = u[e];
+          g.C2[(int64_t)b * g.sc + at] = make_double2(v[e].x + g.beta[3] * u[e].x, v[e].y + g.beta[3] * u[e].y);
+        } else {
+          C[at] = v[e];
+        }
+      }
+    }
+}
+
+__device__ __forceinline__ int zg_size(const ZGemm& g, int b) { return g.own.nns ? g.own.nns[g.own.dirs[b]] : g.own.n ? g.own.n : 1 << 30; }
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_zgemm(ZGemm g) {
+  __shared__ __attribute__((aligned(1024))) double2 lds[2048];
+  const int tm = (g.m + 63) / 64, tn = (g.n + 63) / 64;
+  // the second results, twice the work of the first, start first
+  const int nblk = tm * tn * g.nb, dual = g.Xd && (int)blockIdx.x < nblk;
+  const int lb = xcd_logical_block((int)blockIdx.x >= nblk ? blockIdx.x - nblk : blockIdx.x, nblk);
+  const int b = lb / (tm * tn), tt = lb % (tm * tn);
+  if (g.active && g.step >= g.active[b]) return;
+  const int n = zg_size(g, b), lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int place = (wave + b + tt) & 3;
+  ZgTile t;
+  t.o = zg_operands(g, dual);
+  t.bm = (tt % tm) * 64; t.bn = (tt / tm) * 64;
+  t.wm = (place >> 1) * 32; t.wn = (place & 1) * 32;
+  t.me = (g.trim & 1) ? min(g.m, n) : g.m;
+  t.ne = (g.trim & 2) ? min(g.n, n) : g.n;
+  t.ke = (g.trim & 4) ? min(g.k, n) : g.k;
+  const int ui = t.me - (t.bm + t.wm), uj = t.ne - (t.bn + t.wn);
+  // (the waves of a workgroup run different copies of the same sequence of barriers)
+  if (ui <= 0 || uj <= 0) zg_run<0, 0>(g, t, b, wave, lane, lds);
+  else if (ui > 16 && uj > 16) zg_run<2, 2>(g, t, b, wave, lane, lds);
+  else if (ui > 16) zg_run<2, 1>(g, t, b, wave, lane, lds);
+  else if (uj > 16) zg_run<1, 2>(g, t, b, wave, lane, lds);
+  else zg_run<1, 1>(g, t, b, wave, lane, lds);
+}
+
+// The same product, in the same order and so with the same result, where 64x64 tiles would leave CUs idle (a
+// few matrices): one workgroup per 16x16 tile, one wave for the real and one for the imaginary part, operands
+// straight from L2. Bound by latency: the serial chain of K/2 MFMAs and the loads ahead of it. A 96 x 96
+// product: 22 -> 12 us.
+__global__ __launch_bounds__(128) void k_zgemm_few(ZGemm g) {
+  const int tm = (g.m + 15) / 16, tn = (g.n + 15) / 16;
+  const int nblk = tm * tn * g.nb, dual = g.Xd && (int)blockIdx.x < nblk;
+  const int lb = (int)blockIdx.x >= nblk ? blockIdx.x - nblk : blockIdx.x;
+  const int b = lb / (tm * tn), tt = lb % (tm * tn);
+  if (g.active && g.step >= g.active[b]) return;
+  const ZgOperands o = zg_operands(g, dual);
+  const int n = zg_size(g, b), lane = threadIdx.x & 63, im = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, l4 = lane >> 4;
+  const int bm = (tt % tm) * 16, bn = (tt / tm) * 16;
+  const int me = (g.trim & 1) ? min(g.m, n) : g.m, ne = (g.trim & 2) ? min(g.n, n) : g.n;
+  const int ke = (bm < me && bn < ne) ? ((g.trim & 4) ? min(g.k, n) : g.k) : 0;
+  const int row = bm + l16;
+  double mv[4][4];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int col = bn + l4 + 4 * e;
+      mv[q][e] = (o.M[q] && row < g.m && col < g.n)
+                     ? ((const double*)(o.M[q] + (int64_t)b * g.sm + (int64_t)col * g.ldm + row))[im] : 0.0;
+    }
+  double4v acc = {0, 0, 0, 0};
+  for (int p = 0; p < o.np; p++) {
+    const double2* X = o.X[p] + (int64_t)b * g.sx + min(row, g.m - 1);
+    const double2* Y = o.Y[p] + (int64_t)b * g.sy + (int64_t)min(bn + l16, g.n - 1) * g.ldy;
+#pragma unroll 8
+    for (int k0 = 0; k0 < ke; k0 += 4) {
+      const int k = k0 + l4, kc = min(k, g.k - 1);
+      double2 x = X[(int64_t)kc * g.ldx], y = Y[kc];
+      if (k >= g.k) x = y = make_double2(0.0, 0.0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(im ? y.y : y.x, x.x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(im ? y.x : y.y, im ? x.y : -x.y, acc, 0, 0, 0);
+    }
+  }
+  if (row >= g.m) return;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int col = bn + l4 + 4 * e;
+    if (col >= g.n) continue;
+    const bool diag = row == col && !im;
+    const int64_t at = 2 * ((int64_t)b * g.sc + (int64_t)col * g.ldc + row) + im;
+    double v = g.alpha * acc[e];
+    if (diag) v += o.betaI;
+    if (g.C2) {
+      ((double*)o.C)[at] = v;
+      mv[3][e] = v;
+      v = diag ? g.betaI2 : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (o.M[q] || (g.C2 && q == 3)) v += g.beta[q] * mv[q][e];
+    ((double*)(g.C2 ? g.C2 : o.C))[at] = v;
+  }
 }
 
 void launch_zgemm(hipStream_t s, const ZGemm& g) {
-  const int tm = (g.m + 63) / 64, tn = (g.n + 63) / 64;
-  hipLaunchKernelGGL(k_zgemm, dim3(tm * tn * g.nb), dim3(256), 0, s, g);
+  const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.nb;
+  const int res = g.Xd ? 2 : 1;
+  if (tiles < kZgemmFew)
+    hipLaunchKernelGGL(k_zgemm_few, dim3(((g.m + 15) / 16) * ((g.n + 15) / 16) * g.nb * res), dim3(128), 0, s, g);
+  else
+    hipLaunchKernelGGL(k_zgemm, dim3((unsigned)(tiles * res)), dim3(256), 0, s, g);
 }
 
 // ------------------------------------------------------------------------------------------
