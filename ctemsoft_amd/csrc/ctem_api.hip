@@ -232,6 +232,7 @@ struct ctem_plan {
   int32_t ecp_nt = 0, ecp_numt = 0;
   float ecp_t0 = 0.0f, ecp_dt = 0.0f, ecp_zint = 0.0f;
   double ecp_nat = 1.0, ecp_s0 = 1.0;
+  DBuf selbits;  // the beam selection's class masks
   DBuf fn, ecp_slut, ecp_store, ecp_thick, ecp_sr, ecp_part;
 };
 
@@ -682,7 +683,7 @@ extern "C" int32_t ctem_plan_destroy(ctem_plan* p) {
     p->ctx->mgraph_key.clear();
   }
   for (DBuf* b : {&p->k, &p->kn, &p->lam, &p->ij, &p->nns, &p->nnw, &p->soff, &p->woff, &p->sidx,
-                  &p->ssg, &p->widx, &p->wsg, &p->err, &p->dots, &p->keep_lgh, &p->dirs, &p->fn, &p->ecp_slut,
+                  &p->ssg, &p->widx, &p->wsg, &p->err, &p->dots, &p->keep_lgh, &p->dirs, &p->selbits, &p->fn, &p->ecp_slut,
                   &p->ecp_store, &p->ecp_thick, &p->ecp_sr, &p->ecp_part})
     b->release();
   p->cr.reset();
@@ -728,6 +729,8 @@ extern "C" int32_t ctem_plan_select(ctem_plan* p, int32_t* nns_out, int32_t* nnw
   o.nns = p->nns.as<int32_t>(); o.nnw = p->nnw.as<int32_t>(); o.err = p->err.as<int32_t>();
   DevRefl R = p->cr->refl();
   const float* fnp = p->fn.p ? p->fn.as<float>() : nullptr;
+  if ((rc = p->selbits.ensure(64 * (size_t)((R.nref + 255) / 256) * (size_t)std::max(nk, 1)))) return rc;
+  o.bits = p->selbits.as<uint64_t>();
   launch_select(s, p->k.as<double>(), nk, R, p->cr->rmt.as<double>(), fnp, o, 0);
   HIPCHK(hipGetLastError());
   if ((rc = check_err_flag(p->err, s, "beam selection"))) return rc;

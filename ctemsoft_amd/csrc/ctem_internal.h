@@ -132,6 +132,7 @@ struct SelectOut {       // per-direction beam sets (CSR over directions)
   int32_t* sidx; float* ssg;
   int32_t* widx; float* wsg;
   int32_t* err;          // set to 1 when an angle leaves the reproduced cosf branch
+  uint64_t* bits;        // [numk][ceil(nref / 256)][4][2] class masks, from the counting to the filling pass
 };
 
 // Beam selection. fill=0 counts, fill=1 writes the lists. fn (float[3] on the device, or null):

@@ -29,76 +29,97 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------------------------------
 // beam selection
 // fn: the foil normal (float32, reciprocal components) shared by all directions, or null for
-// FN = k of each direction
+// FN = k of each direction. One workgroup per direction, 64 reflections per wave and step, no barriers in the
+// loop. The counting pass (fill = 0) leaves each wave's two class masks in out.bits; the filling pass computes s_g
+// only for the beams that are set there. Bound by the program's acosf/cosf arithmetic of the counting pass.
+// bcc Fe, 21,000 directions: both passes 1.34 -> 0.77 ms against computing s_g twice with three barriers a step.
+template <bool FILL>
 __global__ __launch_bounds__(256) void k_select(const double* __restrict__ kvec, int32_t numk,
                                                 DevRefl R, const double* __restrict__ rmt_g,
-                                                const float* __restrict__ fn_g, SelectOut out, int fill) {
+                                                const float* __restrict__ fn_g, SelectOut out) {
   const int ik = blockIdx.x;
   if (ik >= numk) return;
   __shared__ double rmt[9];
-  __shared__ int wave_s[4], wave_w[4];
-  __shared__ int base_s, base_w;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ int cnt[2][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid < 9) rmt[tid] = rmt_g[tid];
-  if (tid == 0) { base_s = 0; base_w = 0; }
   __syncthreads();
   const float k[3] = {(float)kvec[3 * ik], (float)kvec[3 * ik + 1], (float)kvec[3 * ik + 2]};
   const float fn[3] = {fn_g ? fn_g[0] : k[0], fn_g ? fn_g[1] : k[1], fn_g ? fn_g[2] : k[2]};
-  const int64_t soff = fill ? out.soff[ik] : 0;
-  const int64_t woff = fill ? out.woff[ik] : 0;
+  const int nch = (R.nref + 255) / 256;
+  uint64_t* bits = out.bits + (int64_t)ik * nch * 8;  // [chunk][wave][strong, weak]
   bool range_ok = true;
-  const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  for (int t0 = 0; t0 < R.nref; t0 += 256) {
-    const int ig = t0 + tid;
-    int cls = 0;
-    float sg = 0.0f;
-    if (ig == 0) {
-      cls = 2;  // the transmitted beam is always strong, with s_g = 0
-    } else if (ig < R.nref) {
-      const float g[3] = {R.g[3 * ig], R.g[3 * ig + 1], R.g[3 * ig + 2]};
-      sg = calcsg_fn(g, k, fn, rmt, &range_ok);
-      const float sgp = fabsf(sg);
-      if (R.dbd[ig]) {
-        if (sgp <= R.sgcutoff) cls = 2;
-      } else if (sgp <= R.cut1[ig]) {
-        cls = (sgp <= R.cut2[ig]) ? 2 : 1;
+  auto sg_of = [&](int ig) __attribute__((always_inline)) {
+    if (ig == 0) return 0.0f;
+    const float g[3] = {R.g[3 * ig], R.g[3 * ig + 1], R.g[3 * ig + 2]};
+    return calcsg_fn(g, k, fn, rmt, &range_ok);
+  };
+  if (!FILL) {
+    int ns = 0, nw = 0;
+    for (int c = 0; c < nch; c++) {
+      const int ig = c * 256 + tid;
+      int cls = 0;
+      if (ig == 0) {
+        cls = 2;  // the transmitted beam is always strong, with s_g = 0
+      } else if (ig < R.nref) {
+        const float sgp = fabsf(sg_of(ig));
+        if (R.dbd[ig]) {
+          if (sgp <= R.sgcutoff) cls = 2;
+        } else if (sgp <= R.cut1[ig]) {
+          cls = (sgp <= R.cut2[ig]) ? 2 : 1;
+        }
+      }
+      const uint64_t bs = __ballot(cls == 2), bw = __ballot(cls == 1);
+      ns += __popcll(bs);
+      nw += __popcll(bw);
+      if (lane == 0) {
+        bits[8 * c + 2 * wave] = bs;
+        bits[8 * c + 2 * wave + 1] = bw;
       }
     }
-    const uint64_t bs = __ballot(cls == 2);
-    const uint64_t bw = __ballot(cls == 1);
-    if (lane == 0) { wave_s[wave] = __popcll(bs); wave_w[wave] = __popcll(bw); }
+    if (lane == 0) { cnt[0][wave] = ns; cnt[1][wave] = nw; }
     __syncthreads();
-    if (fill) {
-      int os = base_s, ow = base_w;
-      for (int w = 0; w < wave; w++) { os += wave_s[w]; ow += wave_w[w]; }
-      if (cls == 2) {
-        const int64_t p = soff + os + __popcll(bs & lt);
+    if (tid == 0) {
+      out.nns[ik] = cnt[0][0] + cnt[0][1] + cnt[0][2] + cnt[0][3];
+      out.nnw[ik] = cnt[1][0] + cnt[1][1] + cnt[1][2] + cnt[1][3];
+    }
+    if (!range_ok) atomicOr(out.err, 1);
+    return;
+  }
+  const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+  int64_t os = out.soff[ik], ow = out.woff[ik];  // before this chunk
+  for (int c = 0; c < nch; c++) {
+    int64_t ps = os, pw = ow;  // before this wave
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const int s = __popcll(bits[8 * c + 2 * w]), v = __popcll(bits[8 * c + 2 * w + 1]);
+      os += s;
+      ow += v;
+      if (w < wave) { ps += s; pw += v; }
+    }
+    const uint64_t bs = bits[8 * c + 2 * wave], bw = bits[8 * c + 2 * wave + 1];
+    if (!(bs | bw)) continue;
+    const int ig = c * 256 + tid;
+    if ((bs | bw) >> lane & 1) {
+      const float sg = sg_of(ig);
+      if (bs >> lane & 1) {
+        const int64_t p = ps + __popcll(bs & lt);
         out.sidx[p] = ig;
         out.ssg[p] = sg;
-      } else if (cls == 1) {
-        const int64_t p = woff + ow + __popcll(bw & lt);
+      } else {
+        const int64_t p = pw + __popcll(bw & lt);
         out.widx[p] = ig;
         out.wsg[p] = sg;
       }
     }
-    __syncthreads();
-    if (tid == 0) {
-      base_s += wave_s[0] + wave_s[1] + wave_s[2] + wave_s[3];
-      base_w += wave_w[0] + wave_w[1] + wave_w[2] + wave_w[3];
-    }
-    __syncthreads();
   }
-  if (!fill && tid == 0) {
-    out.nns[ik] = base_s;
-    out.nnw[ik] = base_w;
-  }
-  if (!range_ok) atomicOr(out.err, 1);
 }
 
 void launch_select(hipStream_t s, const double* k, int32_t numk, const DevRefl& R,
                    const double* rmt9, const float* fn, const SelectOut& out, int fill) {
   if (numk <= 0) return;
-  hipLaunchKernelGGL(k_select, dim3(numk), dim3(256), 0, s, k, numk, R, rmt9, fn, out, fill);
+  if (fill) hipLaunchKernelGGL(k_select<true>, dim3(numk), dim3(256), 0, s, k, numk, R, rmt9, fn, out);
+  else hipLaunchKernelGGL(k_select<false>, dim3(numk), dim3(256), 0, s, k, numk, R, rmt9, fn, out);
 }
 
 // ------------------------------------------------------------------------------------------
