@@ -618,6 +618,7 @@ void launch_adj_hm(hipStream_t s, int npad, int nb, int nz, const double2* Psi, 
 }
 void launch_adj_depth(hipStream_t s, int npad, int nb, int nz, const double2* E, const double2* Q,
                       const double* lam, double2* Phi) {
+  if (launch_depth_back(s, npad, nb, nz, E, Q, lam, Phi)) return;
   hipLaunchKernelGGL(k_adj_depth, dim3(nb), dim3(256), 2 * npad * sizeof(double2), s, npad, nz, E, Q, lam, Phi);
 }
 void launch_adj_pair(hipStream_t s, int npad, int nb, const double2* A, const double2* Ebar, double* sigma,

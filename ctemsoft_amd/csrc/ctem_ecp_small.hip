@@ -44,14 +44,6 @@ __device__ __forceinline__ double lane_of(double v, int l) {  // lane l's v, in 
   return __longlong_as_double(((uint64_t)hi << 32) | lo);
 }
 
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-  const uint64_t u = __double_as_longlong(v);
-  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
-  const uint32_t hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((uint64_t)hi << 32) | lo);
-}
-
 // max over the workgroup, the same in every thread (a NaN wins); red: four doubles of LDS
 __device__ __forceinline__ double block_max(double v, double* red) {
   auto mx = [](double a, double b) { return (a != a) ? a : ((b != b) ? b : fmax(a, b)); };
@@ -132,9 +124,9 @@ struct Wg {
       cmac(x, X[c * LD + r], v);
       cmac(y, Y[c * LD + r], CONJ ? make_double2(v.x, -v.y) : v);
     }
-    x.x += dpp<0xb1>(x.x); x.y += dpp<0xb1>(x.y);  // quad_perm [1,0,3,2]
-    x.x += dpp<0x4e>(x.x); x.y += dpp<0x4e>(x.y);  // quad_perm [2,3,0,1]
-    if (G == 8) { x.x += dpp<0x141>(x.x); x.y += dpp<0x141>(x.y); }  // row_half_mirror
+    x.x += dpp_f64<0xb1>(x.x); x.y += dpp_f64<0xb1>(x.y);  // quad_perm [1,0,3,2]
+    x.x += dpp_f64<0x4e>(x.x); x.y += dpp_f64<0x4e>(x.y);  // quad_perm [2,3,0,1]
+    if (G == 8) { x.x += dpp_f64<0x141>(x.x); x.y += dpp_f64<0x141>(x.y); }  // row_half_mirror
   }
   static constexpr size_t lds() { return (size_t)(2 * NP * LD + 2 * NP) * sizeof(double2) + 64 * sizeof(double); }
 };

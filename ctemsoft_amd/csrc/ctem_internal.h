@@ -228,6 +228,9 @@ void launch_parity_copy(hipStream_t s, int32_t npad, int32_t nb, const int32_t* 
 // add_identity is set. grid = number of persistent workgroups (normally the CU count).
 void launch_depth(hipStream_t s, int32_t npad, int32_t nb, int32_t nz, const void* E, int fp32,
                   int add_identity, double2* Psi, int64_t spsi, int32_t grid);
+// phi_Z = lam_Z Q_Z, phi_k = lam_k Q_k + E^H phi_{k+1} with E on chip (up to 128 beams); false: too large, nothing done
+bool launch_depth_back(hipStream_t s, int32_t npad, int32_t nb, int32_t nz, const double2* E, const double2* Q,
+                       const double* lam, double2* Phi);
 // the depth recursion from F = E - I and F2 = E^2 - I (FP32, column-major): psi_1 = E e_1,
 // psi_2 = E psi_1, then psi_{k+2} = E^2 psi_k for two depths per pass over F2
 void launch_depth_quad(hipStream_t s, int32_t npad, int32_t nb, int32_t nz, const float2* F, const float2* F2,
