@@ -335,9 +335,8 @@ __global__ __launch_bounds__(256) void k_pade_accum(int npad, int icnt, const in
 }
 
 // X <- D^-1 X for each matrix (npad x npad, column-major): Gauss-Jordan elimination with partial
-// pivoting (largest |re| + |im| in the column, the first of equals). With onchip (npad <= 64) the
-// two matrices are held in LDS for the elimination. err bit 2: a zero pivot.
-__global__ __launch_bounds__(256) void k_zsolve(int n, double2* __restrict__ Dg, double2* __restrict__ Xg, int onchip,
+// pivoting (largest |re| + |im| in the column, the first of equals). err bit 2: a zero pivot.
+__global__ __launch_bounds__(256) void k_zsolve(int n, double2* __restrict__ Dg, double2* __restrict__ Xg,
                                                 int32_t* __restrict__ err) {
   extern __shared__ double2 sh[];
   const int b = blockIdx.x;
@@ -348,13 +347,6 @@ __global__ __launch_bounds__(256) void k_zsolve(int n, double2* __restrict__ Dg,
   double2* D = Dg + b * per;
   double2* X = Xg + b * per;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (onchip) {
-    double2* Dl = sh + 3 * n;
-    double2* Xl = Dl + per;
-    for (int64_t e = tid; e < per; e += 256) { Dl[e] = D[e]; Xl[e] = X[e]; }
-    D = Dl;
-    X = Xl;
-  }
   __shared__ double rv[4];
   __shared__ int ri[4];
   __shared__ int piv_s;
@@ -437,9 +429,6 @@ __global__ __launch_bounds__(256) void k_zsolve(int n, double2* __restrict__ Dg,
       X[e] = v;
     }
   }
-  __syncthreads();
-  if (onchip)
-    for (int64_t e = tid; e < per; e += 256) Xg[b * per + e] = X[e];
 }
 
 void launch_pade_prep(hipStream_t s, int32_t npad, int32_t nb, double2* A, double2* N, double2* D, double2* C,
@@ -455,9 +444,8 @@ void launch_pade_accum(hipStream_t s, int32_t npad, int32_t nb, int32_t icnt, co
 }
 
 void launch_zsolve(hipStream_t s, int32_t npad, int32_t nb, double2* D, double2* X, int32_t* err) {
-  const int onchip = npad <= 64 ? 1 : 0;
-  const size_t lds = (size_t)3 * npad * sizeof(double2) + (onchip ? (size_t)2 * npad * npad * sizeof(double2) : 0);
-  hipLaunchKernelGGL(k_zsolve, dim3(nb), dim3(256), lds, s, npad, D, X, onchip, err);
+  const size_t lds = (size_t)3 * npad * sizeof(double2);
+  hipLaunchKernelGGL(k_zsolve, dim3(nb), dim3(256), lds, s, npad, D, X, err);
 }
 
 void launch_ecp_depth_dots(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
