@@ -1490,10 +1490,13 @@ static void alg_flops(int n, int w, int nz, int nsite, double amod, double /*dz*
 
 namespace {
 
-// form of the matrix exponential a run uses (the squaring counts differ between forms)
+// form of the matrix exponential a run uses, for a plan with its crystal: 0 FP64, 1 split FP16, 2 split BF16, 3 split
+// FP16 on complex-symmetric matrices (inversion-symmetric LUT). The squaring counts differ between
+// them (the norm bounds do), and are kept by form.
 int run_form(const ctem_plan* p, int32_t precision) {
   if (precision == CTEM_PREC_FP64) return 0;
-  return (p->terms_taylor == CTEM_SPLIT_FP16X3 && p->terms_square == CTEM_SPLIT_FP16X3) ? 1 : 2;
+  if (p->terms_taylor != CTEM_SPLIT_FP16X3 || p->terms_square != CTEM_SPLIT_FP16X3) return 2;
+  return p->symmetry == 1 && p->cr->centro ? 3 : 1;
 }
 
 size_t chunk_budget(const ctem_plan* p) { return p->chunk_bytes; }
@@ -1570,9 +1573,8 @@ int32_t run_enqueue(ctem_plan* p, int32_t precision, bool timed, bool sync_ok, d
       Bucket B{npad, nb, p->dirs.as<int32_t>() + off + c0};
       std::vector<int> hn(nb);
       for (int b = 0; b < nb; b++) hn[b] = p->h_nns[kv.second[c0 + b]];
-      const bool split = form == 1;
-      // complex-symmetric DynMat (inversion-symmetric LUT): upper tiles only, split form alone
-      const bool sym = split && p->symmetry == 1 && p->cr->centro;
+      // symmetric: upper tiles only
+      const bool sym = form == 3, split = form == 1 || sym;
       float* amax = nullptr;
       if (precision == CTEM_PREC_MIXED) {
         // six maxima and six exponents per matrix for the products, then the max of A
@@ -1928,10 +1930,10 @@ static int32_t plan_adjoint(ctem_plan* p, bool mixed, const double* gdots, doubl
   LdB.slut = p->cr->st->dslut.as<double2>();
   const double dzt = p->dz / p->thick;
   const int form = run_form(p, CTEM_PREC_MIXED);
-  const bool split = mixed && form == 1;
+  const bool split = mixed && form != 2;
   // (its forward keeps the degree-8 polynomial's products: B's gradient is one sum over every direction, as
   // far from the 64-bit value as its rounding happens to fall, and is not moved by a rounding of another kind)
-  const bool sym = split && p->symmetry == 1 && p->cr->centro;
+  const bool sym = split && form == 3;
   const size_t budget = (size_t)16 << 30;
   size_t off = 0;
   std::vector<int32_t> h_sq, h_sq2;

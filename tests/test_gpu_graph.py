@@ -111,3 +111,32 @@ def test_autotune_picks_and_caches(ctx, tmp_path, monkeypatch):
     plan.run("fp64")
     assert np.allclose(plan.dots(), ref, rtol=1e-12, atol=0)
     plan.close()
+
+
+@pytest.mark.parametrize("weak", [4.0, 30.0, 100.0])
+def test_series_after_symmetry_change(ctx, weak):
+    """The squaring counts kept from one exponential are not taken for another: a plan run with full products
+    and then with symmetric ones (whose polynomial has a smaller norm bound and so more squarings) goes through
+    the captured series, there and back, with the eager run's bits."""
+    from ctemsoft_amd import ebsd, workloads, xtal
+    wl = workloads.get("fe_c1")
+    st, _ = xtal.native_setup(wl.xtal, wl.ekev, wl.dmin, (weak, 2.0 * weak, 0.05))
+    npx, npy = ebsd.lambert_dims(8, st.usehex)
+    _, k, kn = ebsd.kvectors(npx, npy, st.isym, st.usehex, st.dsm, st.mlambda)
+    lam = np.exp(-np.arange(1, 11) / 8.0).astype(np.float32)
+    ctx.upload_crystal(st)
+    ref = {}
+    for on in (0, 1):
+        p = ctx.plan(k, kn, lam, 1.0, 10.0)
+        p.set_symmetry(on)
+        p.run("mixed")
+        ref[on] = p.dots().copy()
+        p.close()
+    for dz in (1.0, 1.3):  # two step lengths: the counts' largest differs in at least one
+        p = ctx.plan(k, kn, lam, dz, 10.0)
+        for on in (0, 1, 0):
+            p.set_symmetry(on)
+            ebsd.run_plans([p], "mixed")
+            if dz == 1.0:
+                assert np.array_equal(p.dots().view(np.int64), ref[on].view(np.int64)), on
+        p.close()
