@@ -290,7 +290,7 @@ def main():
                      "peak": PEAK[head] / 1e12, "unit": "TFLOP/s",
                      "frac": None if ach is None else round(ach * 1e12 / PEAK[head], 4),
                      "traffic": measured_traffic(wl.name, head),
-                     "kernel": "k_zgemm" if head == "fp64" else ("k_expm_sym, k_sym or k_sgemm" if a.terms == "16,16" else "k_cgemm"),
+                     "kernel": "k_zgemm" if head == "fp64" else ("k_expm_sym or k_sgemm" if a.terms == "16,16" else "k_cgemm"),
                      "alg_flops_per_step": alg["products"] if "fp64" in res else None,
                      "kernel_ms_per_step": round(r["gemm"]["gemm_ms"], 3),
                      "kernel_ms_source": ("HIP events of an eager pass after the timed graph steps"

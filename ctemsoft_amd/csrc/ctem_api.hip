@@ -1139,10 +1139,9 @@ SymCoef sym_coef() {
 // 2e-7, 5e-7 and 4e-9; at 1.07 it would be 1e-6 to 3e-6
 constexpr double kThetaSym = 0.9;
 
-// The complex-symmetric form of expm_depth_split, for the sizes that sym_tiles accepts. Buffers (8 bytes
-// per entry): 0 A as assembled, 1 Q1, 2 Q3 (or the tile images that do not fit on chip), 3 the FP32
-// F for the depth kernel, 4 and 5 the squarings, 6 and 7 E^2 - I and E^4 - I. wmax holds maxima and
-// exponents as in expm_depth_split.
+// The complex-symmetric form of expm_depth_split, for the sizes that sym_onchip accepts. Buffers (8 bytes
+// per entry): 0 A as assembled, 1 Q1's terms, 2 the tile images that do not fit on chip, 3 the FP32 F for the
+// depth kernel. wmax holds maxima and exponents as in expm_depth_split.
 int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
                        const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz, int32_t* d_sq,
                        int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq, int depth_grid,
@@ -1169,71 +1168,15 @@ int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W
   // flops of one symmetric product: the entries on and above the diagonal
   auto pflops = [&](int b) { return 4.0 * h_n[b] * h_n[b] * (h_n[b] + 1.0); };
   float2* Ff = W32 + 3 * per * nb;
-  if (sym_onchip(npad)) {
-    double fl = 0.0;
-    for (int b = 0; b < nb; b++) fl += (3 + h_sq[b]) * pflops(b);
-    GemmTimer t{tp, s};
-    t.begin();
-    launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
-    t.end();
-    HIPCHK(hipGetLastError());
-    if (tp) { tp->f_gemm += fl; tp->n_gemm++; }
-    launch_depth(s, npad, nb, nz, Ff, 1, 1, Psi64, spsi, depth_grid);
-    HIPCHK(hipGetLastError());
-    return CTEM_OK;
-  }
-  auto launch = [&](const SymGemm& g, double flops) -> int32_t {
-    GemmTimer t{tp, s};
-    t.begin();
-    launch_sym(s, g);
-    t.end();
-    HIPCHK(hipGetLastError());
-    if (tp) { tp->f_gemm += flops; tp->n_gemm++; }
-    return CTEM_OK;
-  };
-  // matrices past 224 are too large for the on-chip depth kernel: two squarings more give E^2 - I and
-  // E^4 - I (FP32, buffers 6 and 7) for the depth recursion over groups of four depths
-  float2* Ff2 = W32 + 6 * per * nb;
-  float2* Ff4 = W32 + 7 * per * nb;
-  const int extra = 2;
-  double f3 = 0.0;
-  for (int b = 0; b < nb; b++) f3 += pflops(b);
-  auto mk = [&](int c, int x) {
-    SymGemm g{};
-    g.n = npad; g.nb = nb;
-    if (x != 0) g.X = S(x);
-    g.xe = ex(x); g.xmax = mx(x);
-    g.A = W32; g.rs = d_sq; g.bmax = mx(0);
-    g.C = S(c); g.ce = ex(c); g.cmax = mx(c);
-    g.alpha = make_float2(1.0f, 0.0f);
-    return g;
-  };
-  auto finals = [&](SymGemm& g, int at) { g.Cf[0] = Ff; g.Cf[1] = Ff2; g.Cf[2] = Ff4; g.f_sq = d_sq; g.f_at = at; };
-  int32_t rc;
-  const int pc[3] = {1, 2, 5}, px[3] = {0, 1, 2};
-  for (int i = 0; i < 3; i++) {
-    SymGemm g = mk(pc[i], px[i]);
-    g.alpha = coef.alpha[i]; g.bx = coef.bx[i];
-    g.bb = coef.bb[i]; g.has_b = i > 0 ? 1 : 0;
-    if (i == 2) { g.Q = S(1); g.qe = ex(1); g.qmax = mx(1); g.bq = coef.bq[i]; finals(g, 0); }
-    if ((rc = launch(g, f3))) return rc;
-  }
-  const int buf[2] = {5, 4};
-  for (int i = 0; i < smax + extra; i++) {
-    double fl = 0.0;
-    for (int b = 0; b < nb; b++) if (i < h_sq[b] + extra) fl += pflops(b);
-    const int x = buf[i & 1], out = buf[(i + 1) & 1];
-    // the output buffer's maxima were those of two steps back
-    launch_fill_zero(s, mx(out), sizeof(float) * (size_t)nb);
-    SymGemm g = mk(out, x);
-    g.bx = make_float2(2.0f, 0.0f);
-    // every matrix of the chunk in the grid; those whose squarings (plus the extra two) are done
-    // leave at once (counts stay on the device)
-    g.active = d_sq; g.step = i; g.active_add = extra;
-    finals(g, i + 1);
-    if ((rc = launch(g, fl))) return rc;
-  }
-  launch_depth_quad(s, npad, nb, nz, Ff, Ff2, Ff4, Psi64, spsi, depth_grid);
+  double fl = 0.0;
+  for (int b = 0; b < nb; b++) fl += (3 + h_sq[b]) * pflops(b);
+  GemmTimer t{tp, s};
+  t.begin();
+  launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
+  t.end();
+  HIPCHK(hipGetLastError());
+  if (tp) { tp->f_gemm += fl; tp->n_gemm++; }
+  launch_depth(s, npad, nb, nz, Ff, 1, 1, Psi64, spsi, depth_grid);
   HIPCHK(hipGetLastError());
   return CTEM_OK;
 }
@@ -1250,7 +1193,7 @@ int32_t expm_depth_split(ctem_plan* tp, hipStream_t s, int npad, int nb, float2*
                          const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz,
                          int32_t* d_sq, int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq,
                          int depth_grid, bool sym, ChunkSched* cs, bool squares = true) {
-  if (sym && squares && sym_tiles(npad))
+  if (sym && squares && sym_onchip(npad))
     return expm_depth_sym(tp, s, npad, nb, W32, colpart, amax, wmax, Psi64, spsi, nz, d_sq, d_err, h_n, h_sq, depth_grid,
                           cs);
   const int64_t per = (int64_t)npad * npad;

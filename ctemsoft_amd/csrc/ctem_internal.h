@@ -329,34 +329,16 @@ struct SGemm {
 void launch_sgemm(hipStream_t s, const SGemm& g);
 
 // ---- complex-symmetric matrices (ctem_sym.hip) ----
-// The polynomial of exp(B) - I by squares (kSymCoef in ctem_api.hip):
+// The polynomial of exp(B) - I by squares (sym_coef in ctem_api.hip):
 //   Q1 = B B + c B,  Q3 = Q1 Q1 + d1 Q1 + d B,  F0 = s Q3 Q3 + e1 Q3 + q Q1 + b B
 // step by step as v = alpha (X X + bx X + bb B + bq Q1)
 struct SymCoef { float2 alpha[3], bx[3], bb[3], bq[3]; };
-// sizes that launch_sym takes, and those that launch_expm_sym takes
-bool sym_tiles(int n);
+// the sizes that launch_expm_sym takes
 bool sym_onchip(int n);
 // F = exp(A) - I (FP32, both triangles) from the assembled A (its tiles on and above the diagonal),
 // squaring counts and exponents of B = A 2^-sq, one launch. Q, spill: work space, n n 8 bytes per matrix.
 void launch_expm_sym(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
                      float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c);
-// One product C = alpha (X X + bx X + bb B + bq Q) over nb matrices in tile images (B = A 2^-rs;
-// with X null, X = B). Maxima and exponents as in SGemm.
-struct SymGemm {
-  int32_t n, nb;
-  const uint16_t* X; const int32_t* xe; const float* xmax;
-  const float2* A; const int32_t* rs; const float* bmax;
-  const uint16_t* Q; const int32_t* qe; const float* qmax;
-  uint16_t* C; int32_t* ce; float* cmax;
-  float2 alpha, bx, bb, bq;
-  int32_t has_b;
-  const int32_t* active; int32_t step, active_add;  // matrices with step >= active[b] + active_add are skipped
-  // FP32 copies of C, both triangles: Cf[t] for the matrices with f_sq[b] + t == f_at (the result and
-  // the two squarings after it); no C is stored after a matrix's last one
-  float2* Cf[3]; const int32_t* f_sq; int32_t f_at;
-};
-void launch_sym(hipStream_t s, const SymGemm& g);
-
 // zero `bytes` bytes (a multiple of 4) of device memory with a kernel (no memset node, so that
 // the sequence can be captured into a graph)
 void launch_fill_zero(hipStream_t s, void* p, size_t bytes);

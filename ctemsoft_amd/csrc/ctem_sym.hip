@@ -5,7 +5,7 @@
 // step are rows of one strip, the matrix at 32 columns k, and every 32 x 32 output tile (i <= j) takes its
 // A operand from the strip's row tile i and its B operand from row tile j, both as 8 consecutive k of
 // one row per lane. The polynomial of the exponential is therefore evaluated by squares only
-// (kSym* below), and a workgroup keeps the whole upper triangle of a product in its accumulators.
+// (sym_coef in ctem_api.hip), and a workgroup keeps the whole upper triangle of a product in its accumulators.
 //
 // Tile image: the 32 x 32 tiles on and above the diagonal, 8 KB each (four planes of 2 KB); a plane
 // holds its 32 columns one after the other, each as four 16-byte chunks of 8 rows, chunk ch of
@@ -17,13 +17,11 @@
 // LDS and accumulators in registers. The tile (i, j) is used in strips i and j only, so at strip k the
 // live tiles are those with i <= k <= j: at most 16 of the 28 at n = 224, and 19 tiles of LDS
 // hold a matrix whose last nine tiles wait in a global buffer until their places are free.
-// k_sym (larger): one product per launch, strips streamed through a ring of LDS tiles, the triangle
-// shared out over equal parts.
 //
 // Measured on one MI355X, the exponentials of a run against k_sgemm's chain (64 x 64 tiles, three general
 // products for a degree-8 polynomial; it moves 2.3 MB to LDS per product at n = 224 and waits for memory):
 // bcc Fe, 63,252 directions of 188-250 beams: 141 -> 91 ms, 9 products per matrix instead of 8; fcc Ni, 1,326 of
-// 87-115: 1.02 -> 0.51 ms; corundum, 4,300 of 264-362: 30.2 -> 26.5 ms. At n = 224 a strip of a squaring takes
+// 87-115: 1.02 -> 0.51 ms. At n = 224 a strip of a squaring takes
 // ~8,100 cycles where its matrix-core work is 5,376 (7 tiles per SIMD); the rest is the wait for LDS after each
 // barrier, and ~16,000 cycles per product between products.
 #include <hip/hip_runtime.h>
@@ -45,7 +43,6 @@ typedef unsigned int u4v __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 4096;   // halfs of a tile image
 constexpr int kPlane = 1024;  // halfs of a plane
-constexpr int kLdsMax = 160 * 1024;
 
 // 1 KB from global memory (lane l's 16 bytes at src + 16 l) to LDS (dst + 16 l; src and dst uniform) by
 // the load unit, asynchronously: the caller waits with s_waitcnt vmcnt(0) before the barrier ahead of the
@@ -517,190 +514,12 @@ void expm_case(hipStream_t s, int nb, int cus, const ExpmArgs& a) {
                      NSL * kTile * sizeof(_Float16) + 64, s, a);
 }
 
-// ---- one product per launch ----------------------------------------------------------------------
-
-// C = alpha (X X + bx X + bb B + bq Q) (complex coefficients; Q in tile images, B from the raw A). One
-// workgroup of eight waves per (matrix, part): at most four tiles per wave.
-template <bool RAW>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sym(SymGemm g, int parts, int nsl) {
-  constexpr int NS = 4, NW = 8;
-  extern __shared__ __attribute__((aligned(16))) _Float16 Ls[];
-  const int n = g.n, T = n >> 5;
-  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int b = lb / parts, part = lb % parts;
-  if (g.active && g.step >= g.active[b] + g.active_add) return;
-  const int64_t per = (int64_t)n * n, mb = (int64_t)b * 4 * per;
-  const _Float16* X = (const _Float16*)g.X + mb;
-  const float2* A32 = g.A + (int64_t)b * per;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l15 = lane & 15, g4 = lane >> 4;
-
-  const int N = T * (T + 1) / 2, W = NW * parts;
-  const int u = part * NW + (wave & 3) * 2 + (wave >> 2);
-  const int t0 = u * N / W, cnt = (u + 1) * N / W - t0;
-  int dummy;
-  const int imin = row_tile(part * NW * N / W, T, dummy);  // the part's rows and columns are imin .. T - 1
-  const int nrow = T - imin;
-  int si[NS], sj[NS];
-#pragma unroll
-  for (int q = 0; q < NS; q++) si[q] = row_tile(min(t0 + q, N - 1), T, sj[q]);
-
-  // strip k takes places (k nrow + r) mod nsl of the ring (base: that of r = 0); row tiles
-  // r0 .. r1 - 1 of a strip are brought in
-  auto ring = [&](int base, int r) __attribute__((always_inline)) {
-    const int p = base + r;
-    return Ls + (p >= nsl ? p - nsl : p) * kTile;
-  };
-  const float fraw = RAW ? ldexpf(1.0f, g.xe[b] - g.rs[b]) : 0.0f;
-  auto stage = [&](int k, int base, int r0, int r1) __attribute__((always_inline)) {
-    if constexpr (RAW) {
-      for (int h = 8 * r0 + wave; h < 8 * r1; h += NW) {
-        const int r = h >> 3, i = imin + r, ti = min(i, k), tj = max(i, k);
-        const int c = 4 * (h & 7) + g4, lr = 2 * l15;
-        const f4v v = *(const f4v*)(A32 + (int64_t)(32 * tj + c) * n + 32 * ti + lr);
-        put_pair(ring(base, r) + chunk_off(c, lr >> 3) + (lr & 7), v, fraw);
-      }
-    } else {
-      for (int h = 8 * r0 + wave; h < 8 * r1; h += NW) {
-        const int r = h >> 3, pc = (h & 7) * 512, i = imin + r, ti = min(i, k), tj = max(i, k);
-        to_lds(X + (int64_t)(tj * (tj + 1) / 2 + ti) * kTile + pc, ring(base, r) + pc, lane);
-      }
-    }
-  };
-
-  Acc acc[NS];
-#pragma unroll
-  for (int q = 0; q < NS; q++) acc[q].zero();
-  const float xmx = g.xmax[b];
-  const int ex = g.xe[b];
-  const float2 fx = make_float2(ldexpf(g.bx.x, ex), ldexpf(g.bx.y, ex));  // (bx / alpha) in accumulator units
-  const Reader rd(lane);
-  const int early = min(nrow, nsl - nrow);  // row tiles of the next strip that fit beside this one
-  stage(0, 0, 0, nrow);
-  for (int k = 0, base = 0; k < T; k++) {
-    const int nbase = base + nrow >= nsl ? base + nrow - nsl : base + nrow;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (k + 1 < T) stage(k + 1, nbase, 0, early);
-    auto tile = [&](int i) __attribute__((always_inline)) { return ring(base, i - imin); };
-    h8v x[2][4];
-#pragma unroll
-    for (int q = 0; q < NS; q++)
-      if (q < cnt) {
-        if (q == 0 || si[q] != si[q > 0 ? q - 1 : 0]) {
-          rd.read(tile(si[q]), 0, si[q] <= k, x[0]);
-          rd.read(tile(si[q]), 1, si[q] <= k, x[1]);
-        }
-        h8v y[2][4];
-        rd.read(tile(sj[q]), 0, sj[q] <= k, y[0]);
-        rd.read(tile(sj[q]), 1, sj[q] <= k, y[1]);
-        acc[q].mma(x, y[0], 0);
-        acc[q].mma(x, y[1], 1);
-        if (sj[q] == k) acc[q].template add_image<false>(tile(si[q]), fx.x, fx.y, l15, g4);
-      }
-    if (k + 1 < T && early < nrow) {
-      __syncthreads();  // every wave is done with the strip
-      stage(k + 1, nbase, early, nrow);
-    }
-    base = nbase;
-  }
-
-  // output exponent from a bound on the entries (the same in every workgroup of the matrix)
-  auto mag = [](float2 v) __attribute__((always_inline)) { return fabsf(v.x) + fabsf(v.y); };
-  float bnd = (float)n * xmx * xmx + mag(g.bx) * xmx;
-  if (g.has_b) bnd += mag(g.bb) * g.bmax[b];
-  if (g.Q) bnd += mag(g.bq) * g.qmax[b];
-  const int ec = f16_scale_exp(mag(g.alpha) * bnd);
-  if (part == 0 && tid == 0) g.ce[b] = ec;
-  float2* Cf = nullptr;
-  bool last = false;
-  for (int t = 0; t < 3; t++)
-    if (g.Cf[t] && g.f_sq[b] + t == g.f_at) {
-      Cf = g.Cf[t] + (int64_t)b * per;
-      last = t == 2 || g.Cf[t + 1] == nullptr;
-    }
-  const float un = ldexpf(1.0f, -2 * ex), sc = ldexpf(1.0f, ec);
-  const float bs = g.has_b ? ldexpf(1.0f, -g.rs[b]) : 0.0f;
-  const float2 bb = make_float2(g.bb.x * bs, g.bb.y * bs);
-  const float qs = g.Q ? ldexpf(1.0f, -g.qe[b]) : 0.0f;
-  const float2 bq = make_float2(g.bq.x * qs, g.bq.y * qs);
-  _Float16* C = (_Float16*)g.C + mb;
-  float vmax = 0.0f;
-#pragma unroll
-  for (int q = 0; q < NS; q++)
-    if (q < cnt) {
-      const int i = si[q], j = sj[q];
-      const int64_t tb = (int64_t)(j * (j + 1) / 2 + i) * kTile;
-#pragma unroll
-      for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          const int row = 32 * i + 16 * a + 4 * g4, col = 32 * j + 16 * c + l15;
-          const int64_t o = tb + chunk_off(16 * c + l15, 2 * a + (g4 >> 1)) + 4 * (g4 & 1);
-          f4v vr, vi;
-#pragma unroll
-          for (int e = 0; e < 4; e++) { vr[e] = acc[q].re[a][c][e] * un; vi[e] = acc[q].im[a][c][e] * un; }
-          if (g.has_b) {
-            const f4v* p = (const f4v*)(A32 + (int64_t)col * n + row);
-            const f4v m0 = p[0], m1 = p[1];
-            const float br[4] = {m0[0], m0[2], m1[0], m1[2]}, bi[4] = {m0[1], m0[3], m1[1], m1[3]};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              vr[e] += bb.x * br[e] - bb.y * bi[e];
-              vi[e] += bb.x * bi[e] + bb.y * br[e];
-            }
-          }
-          if (g.Q) {
-            const _Float16* Mq = (const _Float16*)g.Q + mb + o;
-            const h4v m0 = *(const h4v*)Mq, m1 = *(const h4v*)(Mq + kPlane);
-            const h4v m2 = *(const h4v*)(Mq + 2 * kPlane), m3 = *(const h4v*)(Mq + 3 * kPlane);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              const float qr = (float)m0[e] + (float)m1[e], qi = (float)m2[e] + (float)m3[e];
-              vr[e] += bq.x * qr - bq.y * qi;
-              vi[e] += bq.x * qi + bq.y * qr;
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const float2 w = cmul(g.alpha, make_float2(vr[e], vi[e]));
-            vr[e] = w.x; vi[e] = w.y;
-          }
-          if (Cf) {
-            f4v* p = (f4v*)(Cf + (int64_t)col * n + row);
-            p[0] = (f4v){vr[0], vi[0], vr[1], vi[1]};
-            p[1] = (f4v){vr[2], vi[2], vr[3], vi[3]};
-            if (i != j)
-#pragma unroll
-              for (int e = 0; e < 4; e++) Cf[(int64_t)(row + e) * n + col] = make_float2(vr[e], vi[e]);
-          }
-          if (!last) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) vmax = fmaxf(vmax, fmaxf(fabsf(vr[e]), fabsf(vi[e])));
-            put_rows(C + o, vr, vi, sc);
-          }
-        }
-    }
-  wave_max_to(vmax, g.cmax + b);
-}
-
 }  // namespace
 
-// Matrices of up to 640: a strip of 20 tile images fills the LDS of a CU.
-bool sym_tiles(int n) { return n <= 640; }
+// Past 224 the operand and the accumulators do not fit on a CU, and k_sgemm's chain is taken: squares streamed
+// through LDS, one product per launch, were up to 7% faster in large batches of 288-352 and 416 beams, up to 9%
+// slower at 256 and 448-640, and 1.3-1.9 times slower for a single direction of any size.
 bool sym_onchip(int n) { return n <= 224; }
-
-void launch_sym(hipStream_t s, const SymGemm& g) {
-  if (g.nb <= 0) return;
-  const int T = g.n / 32, N = T * (T + 1) / 2;
-  const int parts = (N + 31) / 32;  // 128 accumulators per lane at most: five tiles per wave spill
-  const int nsl = std::min(2 * T, kLdsMax / (int)(kTile * sizeof(_Float16)));
-  const size_t lds = (size_t)nsl * kTile * sizeof(_Float16);
-  const dim3 grid(parts * g.nb), blk(512);
-  if (g.X) hipLaunchKernelGGL(k_sym<false>, grid, blk, lds, s, g, parts, nsl);
-  else hipLaunchKernelGGL(k_sym<true>, grid, blk, lds, s, g, parts, nsl);
-}
 
 // One, two, three and four-tile matrices: several workgroups per CU share the matrix cores; from
 // five tiles on one workgroup of eight waves fills the CU.
