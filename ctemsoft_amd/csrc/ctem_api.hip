@@ -22,6 +22,7 @@
 #include "ctem_internal.h"
 #include "ctem_laue.h"
 #include "ctem_sg.h"
+#include "ctem_symcoef.h"
 
 using namespace ctem;
 
@@ -1113,40 +1114,16 @@ int32_t expm_depth_mixed(ctem_plan* tp, hipStream_t s, int npad, int nb, float2*
   return CTEM_OK;
 }
 
-// The polynomial of the complex-symmetric form: with squares only, a product needs one operand on chip
-// (ctem_sym.hip). p(B) = s Q3^2 + e1 W2 + e2 B^2 + B with W2 = (B^2 + c B)^2 and Q3 = W2 + d1 B^2 + d2 B
-// matches exp(B) - I through B^7 when c solves c^4 - 10 c^3 + 39 c^2 - 72 c + 60 = 0 (no real root;
-// this one has the smallest coefficients), with 1/s = 20160 c, D = d1 + c^2 = 14 c - 2 c^2,
-// d2 = 84 c - 2 c D, e1 = 1/24 - s (D^2 + 4 c d2), e2 = 1/2 - s d2^2 - e1 c^2; its B^8 coefficient is off by 0.73
-// of 1/8!. theta: see kThetaSym.
-SymCoef sym_coef() {
-  typedef std::complex<double> C;
-  C c(1.5347072799060086, 1.4831613630292302);
-  for (int i = 0; i < 4; i++) {  // to the last bit by Newton's iteration
-    const C p = (((c - 10.0) * c + 39.0) * c - 72.0) * c + 60.0, dp = ((4.0 * c - 30.0) * c + 78.0) * c - 72.0;
-    c -= p / dp;
-  }
-  const C sc = 1.0 / (20160.0 * c), D = 14.0 * c - 2.0 * c * c, d1 = D - c * c, d2 = 84.0 * c - 2.0 * c * D;
-  const C e1 = 1.0 / 24.0 - sc * (D * D + 4.0 * c * d2), e2 = 0.5 - sc * d2 * d2 - e1 * c * c;
-  auto f = [](C v) { return make_float2((float)v.real(), (float)v.imag()); };
-  const float2 zero = make_float2(0.0f, 0.0f), one = make_float2(1.0f, 0.0f);
-  const C bq = e2 - e1 * d1;
-  return SymCoef{{one, one, f(sc)}, {f(c), f(d1), f(e1 / sc)}, {zero, f(d2 - c * d1), f((1.0 - e1 * d2 - c * bq) / sc)},
-                 {zero, zero, f(bq / sc)}};
-}
-// ||B||_1 bound of that polynomial: the truncation adds 2e-8 to the intensities of bcc Fe and fcc Ni (rms
-// over sampled directions in FP64 arithmetic) and 9e-8 on corundum, where degree 8 at theta = 5/4 adds
-// 2e-7, 5e-7 and 4e-9; at 1.07 it would be 1e-6 to 3e-6
-constexpr double kThetaSym = 0.9;
-
 // The complex-symmetric form of expm_depth_split, for the sizes that sym_onchip accepts. Buffers (8 bytes
-// per entry): 0 A as assembled, 1 Q1's terms, 2 the tile images that do not fit on chip, 3 the FP32 F for the
+// per entry): 0 A as assembled, 1 B^2, 2 the tile images that do not fit on chip, 3 the FP32 F for the
 // depth kernel. wmax holds maxima and exponents as in expm_depth_split.
 int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
                        const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz, int32_t* d_sq,
                        int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq, int depth_grid,
                        ChunkSched* cs) {
-  static const SymCoef coef = sym_coef();
+  static const SymPoly poly = sym_poly();
+  auto f2 = [](const float* v) { return make_float2(v[0], v[1]); };
+  const SymCoef coef{f2(poly.c), f2(poly.d1), f2(poly.d2), f2(poly.r), f2(poly.e1), f2(poly.g)};
   const int64_t per = (int64_t)npad * npad;
   auto S = [&](int i) { return (uint16_t*)(W32 + i * per * nb); };
   auto mx = [&](int i) { return wmax + i * nb; };
@@ -1172,7 +1149,7 @@ int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W
   for (int b = 0; b < nb; b++) fl += (3 + h_sq[b]) * pflops(b);
   GemmTimer t{tp, s};
   t.begin();
-  launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
+  launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), mx(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
   t.end();
   HIPCHK(hipGetLastError());
   if (tp) { tp->f_gemm += fl; tp->n_gemm++; }

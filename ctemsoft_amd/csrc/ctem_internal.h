@@ -329,16 +329,14 @@ struct SGemm {
 void launch_sgemm(hipStream_t s, const SGemm& g);
 
 // ---- complex-symmetric matrices (ctem_sym.hip) ----
-// The polynomial of exp(B) - I by squares (sym_coef in ctem_api.hip):
-//   Q1 = B B + c B,  Q3 = Q1 Q1 + d1 Q1 + d B,  F0 = s Q3 Q3 + e1 Q3 + q Q1 + b B
-// step by step as v = alpha (X X + bx X + bb B + bq Q1)
-struct SymCoef { float2 alpha[3], bx[3], bb[3], bq[3]; };
+// the polynomial of exp(B) - I by squares (ctem_symcoef.h)
+struct SymCoef { float2 c, d1, d2, r, e1, g; };
 // the sizes that launch_expm_sym takes
 bool sym_onchip(int n);
 // F = exp(A) - I (FP32, both triangles) from the assembled A (its tiles on and above the diagonal),
-// squaring counts and exponents of B = A 2^-sq, one launch. Q, spill: work space, n n 8 bytes per matrix.
+// squaring counts, exponents and maxima of B = A 2^-sq, one launch. Q, spill: work space, n n 8 bytes per matrix.
 void launch_expm_sym(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
-                     float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c);
+                     const float* bmax, float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c);
 // zero `bytes` bytes (a multiple of 4) of device memory with a kernel (no memset node, so that
 // the sequence can be captured into a graph)
 void launch_fill_zero(hipStream_t s, void* p, size_t bytes);

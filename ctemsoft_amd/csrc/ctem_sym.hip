@@ -5,7 +5,7 @@
 // step are rows of one strip, the matrix at 32 columns k, and every 32 x 32 output tile (i <= j) takes its
 // A operand from the strip's row tile i and its B operand from row tile j, both as 8 consecutive k of
 // one row per lane. The polynomial of the exponential is therefore evaluated by squares only
-// (sym_coef in ctem_api.hip), and a workgroup keeps the whole upper triangle of a product in its accumulators.
+// (ctem_symcoef.h), and a workgroup keeps the whole upper triangle of a product in its accumulators.
 //
 // Tile image: the 32 x 32 tiles on and above the diagonal, 8 KB each (four planes of 2 KB); a plane
 // holds its 32 columns one after the other, each as four 16-byte chunks of 8 rows, chunk ch of
@@ -16,14 +16,17 @@
 // k_expm_sym (up to 224 beams): one workgroup per matrix does the whole exponential, operands in
 // LDS and accumulators in registers. The tile (i, j) is used in strips i and j only, so at strip k the
 // live tiles are those with i <= k <= j: at most 16 of the 28 at n = 224, and 19 tiles of LDS
-// hold a matrix whose last nine tiles wait in a global buffer until their places are free.
+// hold a matrix whose last nine tiles wait in a global buffer until their places are free. A is read in each of the
+// polynomial's three steps, B^2 written and read back, and at six and seven tiles a side some registers spill.
+// Only the operands are rounded to 22 bits: every other term, 2 X of a squaring included, stays FP32 in the accumulators,
+// and B enters the polynomial exactly. Symmetry is used between different tiles only, with the diagonal tiles read as
+// rows for one operand and as columns for the other.
 //
 // Measured on one MI355X, the exponentials of a run against k_sgemm's chain (64 x 64 tiles, three general
 // products for a degree-8 polynomial; it moves 2.3 MB to LDS per product at n = 224 and waits for memory):
-// bcc Fe, 63,252 directions of 188-250 beams: 141 -> 91 ms, 9 products per matrix instead of 8; fcc Ni, 1,326 of
-// 87-115: 1.02 -> 0.51 ms. At n = 224 a strip of a squaring takes
-// ~8,100 cycles where its matrix-core work is 5,376 (7 tiles per SIMD); the rest is the wait for LDS after each
-// barrier, and ~16,000 cycles per product between products.
+// bcc Fe, 63,252 directions of 188-250 beams: 142 -> 87 ms, with 9-10 products per matrix instead of 8; fcc Ni, 1,326 of
+// 87-115: 1.03 -> 0.48 ms. Intensities against 64 bits over 140 drawn sets: the 2-norm error is 0.57-0.72 of that chain's
+// on average at every size, at most 1.13 of it.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include "ctem_ebsd.h"
@@ -57,24 +60,6 @@ __device__ __forceinline__ void to_lds(const _Float16* src, const _Float16* dst,
 __device__ __forceinline__ int chunk_off(int c, int chunk) {
   const int q = (c >> 2) & 3, f = (q >> 1) | (((q ^ (q >> 1)) & 1) << 1);
   return c * 32 + ((chunk ^ f) << 3);
-}
-
-__device__ __forceinline__ void split2(float s, _Float16& hi, _Float16& lo) {
-  hi = (_Float16)s;
-  lo = (_Float16)(s - (float)hi);
-}
-
-// two FP32 complex entries of one column (re, im, re, im), scaled, into the four planes at dst
-__device__ __forceinline__ void put_pair(_Float16* dst, const f4v& r, float f) {
-  h2v o[4];
-#pragma unroll
-  for (int t = 0; t < 2; t++) {
-    _Float16 h, l;
-    split2(r[2 * t] * f, h, l); o[0][t] = h; o[1][t] = l;
-    split2(r[2 * t + 1] * f, h, l); o[2][t] = h; o[3][t] = l;
-  }
-#pragma unroll
-  for (int p = 0; p < 4; p++) *(h2v*)(dst + p * kPlane) = o[p];
 }
 
 // four consecutive rows (half a chunk) of one column, times sc, into the four planes at dst
@@ -158,35 +143,6 @@ struct Acc {
 #pragma unroll
     for (int a = 0; a < 2; a++) { re[a][c] += r[a]; im[a][c] += i[a]; }
   }
-  // += f X for the tile image at t (stored units)
-  template <bool REAL>
-  __device__ __forceinline__ void add_image(const _Float16* t, float fr, float fi, int l15, int g) {
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const _Float16* o = t + chunk_off(16 * c + l15, 2 * a + (g >> 1)) + 4 * (g & 1);
-        const h4v p0 = *(const h4v*)o, p1 = *(const h4v*)(o + kPlane);
-        const h4v p2 = *(const h4v*)(o + 2 * kPlane), p3 = *(const h4v*)(o + 3 * kPlane);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          float r = __builtin_fmaf(fr, (float)p1[e], re[a][c][e]), i = __builtin_fmaf(fr, (float)p3[e], im[a][c][e]);
-          if (!REAL) {
-            r = __builtin_fmaf(-fi, (float)p3[e], r);
-            i = __builtin_fmaf(fi, (float)p1[e], i);
-          }
-          r = __builtin_fmaf(fr, (float)p0[e], r);
-          i = __builtin_fmaf(fr, (float)p2[e], i);
-          if (!REAL) {
-            r = __builtin_fmaf(-fi, (float)p2[e], r);
-            i = __builtin_fmaf(fi, (float)p0[e], i);
-          }
-          re[a][c][e] = r;
-          im[a][c][e] = i;
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one subtile's planes in registers at a time
-      }
-  }
 };
 
 // tile t of the upper triangle in row order (row i: (i, i) .. (i, T - 1))
@@ -197,7 +153,12 @@ __device__ __forceinline__ int row_tile(int t, int T, int& j) {
   return i;
 }
 
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
+  return make_float2(__builtin_fmaf(-a.y, b.y, a.x * b.x), __builtin_fmaf(a.y, b.x, a.x * b.y));
+}
+__device__ __forceinline__ float2 cmac(float2 s, float2 a, float2 b) {  // s + a b
+  return make_float2(__builtin_fmaf(-a.y, b.y, __builtin_fmaf(a.x, b.x, s.x)), __builtin_fmaf(a.y, b.x, __builtin_fmaf(a.x, b.y, s.y)));
+}
 
 // ---- the whole exponential on chip ------------------------------------------------------------
 
@@ -205,9 +166,10 @@ struct ExpmArgs {
   const float2* A;      // [nb][n n] assembled matrices (column-major FP32; tiles on and above the diagonal)
   const int32_t* sq;    // squaring counts, exponents of B = A 2^-s
   const int32_t* bexp;
+  const float* bmax;    // max |component| of B
   int32_t nb;
   float2* F;            // [nb][n n] out: exp(A) - I, both triangles
-  float* Q;             // [workgroups][N 2048] work: the terms of step 2 in B and Q1, FP32
+  float* Q;             // [workgroups][N 2048] work: B^2, FP32
   _Float16* spill;      // [workgroups][...] work: tile images that do not fit in LDS; strides of both in bytes: n n 8
   SymCoef c;
 };
@@ -258,68 +220,25 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
   const int s = g.sq[b];
   const float bscale = ldexpf(1.0f, -s);
   int ex = g.bexp[b];
-  // B into tile images: two rows of one column per lane, an eighth of a tile (four columns) per wave and
-  // turn, the loads of several turns in flight
-  {
-    constexpr int HT = 8 * N / NW, AT = HT < 14 ? HT : 14;
-    const float f = ldexpf(bscale, ex);
-    const int lr = 2 * l15;
-#pragma unroll 1
-    for (int m0 = 0; m0 < HT; m0 += AT) {
-      f4v v[AT];
-#pragma unroll
-      for (int m = 0; m < AT; m++) {
-        const int h = min(wave + (m0 + m) * NW, 8 * N - 1);
-        int j;
-        const int i = row_tile(h >> 3, T, j);
-        v[m] = *(const f4v*)(A + (int64_t)(32 * j + 4 * (h & 7) + g4) * n + 32 * i + lr);
-      }
-#pragma unroll
-      for (int m = 0; m < AT; m++) {
-        const int h = wave + (m0 + m) * NW, r = h >> 3;
-        if (h >= 8 * N) break;
-        _Float16* dst = (N > NSL && r >= NSL) ? spill + (r - NSL) * kTile : Ls + r * kTile;
-        put_pair(dst + chunk_off(4 * (h & 7) + g4, lr >> 3) + (lr & 7), v[m], f);
-      }
-    }
-  }
-
   const Reader rd(lane);
   Acc acc[NS];
   float un = 1.0f;  // accumulator units 2^(-2 ex)
-  // one product, v = alpha (X X + bx X + bb B + bq Q1): steps 0 to 2 of the polynomial, 3 a squaring. Code of
-  // its own for each, so that nothing but the products decides what becomes of the accumulators.
+  // one product on top of the other terms that next_operand left in the accumulators (of a squaring X, of which it
+  // takes 2 X). Code of its own for each step, so that nothing but the products decides what becomes of the
+  // accumulators.
   auto product = [&](auto st) __attribute__((always_inline)) {
     constexpr int ST = decltype(st)::value;
-    const float up = ldexpf(1.0f, 2 * ex);
+    const float up = ldexpf(1.0f, 2 * ex), carry = ST == 3 ? 2.0f * un * up : up;
     un = ldexpf(1.0f, -2 * ex);
-    float2 fx = ST < 3 ? g.c.bx[ST < 3 ? ST : 0] : make_float2(2.0f, 0.0f);
-    fx.x = ldexpf(fx.x, ex);
-    fx.y = ldexpf(fx.y, ex);
-    if constexpr (ST == 1 || ST == 2) {
-      // the accumulators hold the terms in B and Q1 (in flight: next_operand asked for them)
-      const float f = ST == 1 ? bscale * up : up;
 #pragma unroll
-      for (int t = 0; t < 4 * NS; t++) {
-        const int q = t >> 2, a = (t >> 1) & 1, c = t & 1;
-        const f4v m0 = acc[q].re[a][c], m1 = acc[q].im[a][c];
-        if constexpr (ST == 2) {
-          acc[q].re[a][c] = m0 * f;
-          acc[q].im[a][c] = m1 * f;
-        } else {
-          const float2 bb = make_float2(g.c.bb[1].x * f, g.c.bb[1].y * f);
+    for (int q = 0; q < NS; q++)
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const float2 y = cmul(bb, e < 2 ? make_float2(m0[2 * e], m0[2 * e + 1]) : make_float2(m1[2 * e - 4], m1[2 * e - 3]));
-            acc[q].re[a][c][e] = y.x;
-            acc[q].im[a][c][e] = y.y;
-          }
+      for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          acc[q].re[a][c] = ST == 0 ? (f4v){0, 0, 0, 0} : acc[q].re[a][c] * carry;
+          acc[q].im[a][c] = ST == 0 ? (f4v){0, 0, 0, 0} : acc[q].im[a][c] * carry;
         }
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < NS; q++) acc[q].zero();
-    }
 #pragma unroll 1
     for (int k = 0; k < T; k++) {
       // strip 0: the tiles are in LDS (stores to the global buffer may still be under way); then those
@@ -352,32 +271,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
             rd.read(t, 1, si[q] <= k, x[1]);
           }
           const _Float16* t = row_at(k, sj[q]);
-          rd.read(t, 0, sj[q] <= k, y[0]);
+          rd.read(t, 0, sj[q] < k, y[0]);
           acc[q].mma(x, y[0], 0);
-          rd.read(t, 1, sj[q] <= k, y[1]);
+          rd.read(t, 1, sj[q] < k, y[1]);
           acc[q].mma(x, y[1], 1);
-          if (sj[q] == k) {
-            const _Float16* t = row_at(k, si[q]);
-            acc[q].template add_image<ST == 3>(t, fx.x, fx.y, l15, g4);
-          }
         }
-    }
-    if constexpr (ST == 2) {  // the other steps have alpha = 1
-#pragma unroll
-      for (int t = 0; t < 4 * NS; t++) {
-        const int q = t >> 2, a = (t >> 1) & 1, c = t & 1;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float2 z = cmul(g.c.alpha[2], make_float2(acc[q].re[a][c][e], acc[q].im[a][c][e]));
-          acc[q].re[a][c][e] = z.x;
-          acc[q].im[a][c][e] = z.y;
-        }
-      }
     }
   };
-  // the accumulators become the next operand, with the exponent from their exact maximum over the
-  // workgroup. Ahead of step 1 the terms of step 2 in B and Q1 go to memory; ahead of steps 1 and 2 the
-  // freed accumulators receive the step's terms.
+  // the next operand, and in the accumulators the next product's other terms (ctem_symcoef.h). 0: B from memory.
+  // 1: B^2 + c B, B^2 to memory. 2: r (W + d2 B), B^2 back. 3: the accumulators. Exponents are from the accumulators'
+  // exact maximum over the workgroup, in steps 1 and 2 by a bound of the sum.
   auto next_operand = [&](auto st) __attribute__((always_inline)) {
     constexpr int ST = decltype(st)::value;
     // the lane's place, opaque to the compiler: it would otherwise keep every address in registers
@@ -385,24 +288,61 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const int l15 = ln & 15, g4 = ln >> 4;
-    auto b_at = [&](int q, int a, int c) __attribute__((always_inline)) {
-      return (const f4v*)(A + (int64_t)(32 * sj[q] + 16 * c + l15) * n + 32 * si[q] + 16 * a + 4 * g4);
+    // four rows of A, (re, im) pairs. The table's U(-g) = U(g) holds to about 1e-8 only; where the assembly's 64 x 64
+    // tiles give both triangles, their mean is taken (the upper one alone costs corundum's sets of 33-64 beams
+    // half of their precision)
+    auto load_b = [&](int q, int a, int c, f4v& m0, f4v& m1) __attribute__((always_inline)) {
+      const int row = 32 * si[q] + 16 * a + 4 * g4, col = 32 * sj[q] + 16 * c + l15;
+      const f4v* p = (const f4v*)(A + (int64_t)col * n + row);
+      m0 = p[0];
+      m1 = p[1];
+      if (T > 1 && sj[q] == si[q] + 1 && !(si[q] & 1)) {
+        const float2* t = A + (int64_t)row * n + col;
+        const float2 t0 = t[0], t1 = t[n], t2 = t[2 * n], t3 = t[3 * n];
+        m0 = 0.5f * (m0 + (f4v){t0.x, t0.y, t1.x, t1.y});
+        m1 = 0.5f * (m1 + (f4v){t2.x, t2.y, t3.x, t3.y});
+      }
     };
     auto z_at = [&](int q, int a, int c) __attribute__((always_inline)) {
       return (f4v*)(Q + (int64_t)min(t0 + q, N - 1) * 2048) + ln * 2 + (2 * a + c) * 128;
     };
+    // tile t0 + q's place of rows 4 g4 .. and column l15 of subtile (a, c)
+    auto image = [&](int q, int a, int c) __attribute__((always_inline)) {
+      const int r = t0 + q;
+      _Float16* t = (N > NSL && r >= NSL) ? spill + (r - NSL) * kTile : Ls + r * kTile;
+      return t + chunk_off(16 * c + l15, 2 * a + (g4 >> 1)) + 4 * (g4 & 1);
+    };
+    if constexpr (ST == 0) {
+#pragma unroll
+      for (int q = 0; q < NS; q++)
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int c = 0; c < 2; c++) load_b(q, a, c, acc[q].re[a][c], acc[q].im[a][c]);
+      const float sc = ldexpf(bscale, ex);
+#pragma unroll
+      for (int q = 0; q < NS; q++) {
+        if (q < cnt)
+#pragma unroll
+          for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+              const f4v m0 = acc[q].re[a][c], m1 = acc[q].im[a][c];
+              put_rows(image(q, a, c), (f4v){m0[0], m0[2], m1[0], m1[2]}, (f4v){m0[1], m0[3], m1[1], m1[3]}, sc);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
     f4v m[2][2][2];
     auto ask = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
       for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-          const f4v* p = b_at(q, a, c);
-          m[a][c][0] = p[0];
-          m[a][c][1] = p[1];
-        }
+        for (int c = 0; c < 2; c++) load_b(q, a, c, m[a][c][0], m[a][c][1]);
     };
-    if constexpr (ST == 1 && NS < 4) ask(0);
+    constexpr bool kB = ST == 1 || ST == 2;
+    if constexpr (kB && NS < 4) ask(0);
     float vmax = 0.0f;
 #pragma unroll
     for (int t = 0; t < 4 * NS; t++) {
@@ -424,55 +364,55 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
     vmax = red[0];
 #pragma unroll
     for (int w = 1; w < NW; w++) vmax = fmaxf(vmax, red[w]);
-    ex = f16_scale_exp(vmax * un);
-    const float sc = ldexpf(un, ex);
-    const float2 bb = make_float2(g.c.bb[2].x * bscale, g.c.bb[2].y * bscale);
-    const float2 bq = make_float2(g.c.bq[2].x * un, g.c.bq[2].y * un);
+    vmax *= un;
+    auto mag = [](float2 v) __attribute__((always_inline)) { return fabsf(v.x) + fabsf(v.y); };
+    const float2 f = ST == 1 ? g.c.c : g.c.d2;
+    if constexpr (ST == 1) vmax += mag(f) * g.bmax[b];
+    if constexpr (ST == 2) vmax = mag(g.c.r) * (vmax + mag(f) * g.bmax[b]);
+    ex = f16_scale_exp(vmax);
+    const float sc = ldexpf(kB ? 1.0f : un, ex);
 #pragma unroll
     for (int q = 0; q < NS; q++) {
-      if constexpr (ST == 1 && NS >= 4) ask(q);  // (asked for one tile ahead, they spill)
+      if constexpr (kB && NS >= 4) ask(q);  // (asked for one tile ahead, they spill)
       if (q < cnt) {
-        const int r = t0 + q;
-        _Float16* dst = (N > NSL && r >= NSL) ? spill + (r - NSL) * kTile : Ls + r * kTile;
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
           for (int c = 0; c < 2; c++) {
-            put_rows(dst + chunk_off(16 * c + l15, 2 * a + (g4 >> 1)) + 4 * (g4 & 1), acc[q].re[a][c], acc[q].im[a][c], sc);
-            if constexpr (ST == 1) {
-              f4v zr, zi;
+            f4v& re = acc[q].re[a][c];
+            f4v& im = acc[q].im[a][c];
+            if constexpr (!kB) {
+              put_rows(image(q, a, c), re, im, sc);
+            } else {
+              f4v* p = z_at(q, a, c);
+              f4v zr, zi, xr, xi;
+              if constexpr (ST == 2) { zr = p[0]; zi = p[1]; }
 #pragma unroll
               for (int e = 0; e < 4; e++) {
-                const float2 y = cmul(bb, make_float2(m[a][c][e >> 1][2 * (e & 1)], m[a][c][e >> 1][2 * (e & 1) + 1]));
-                const float2 z = cmul(bq, make_float2(acc[q].re[a][c][e], acc[q].im[a][c][e]));
-                zr[e] = y.x + z.x;
-                zi[e] = y.y + z.y;
+                const float2 B = make_float2(m[a][c][e >> 1][2 * (e & 1)] * bscale, m[a][c][e >> 1][2 * (e & 1) + 1] * bscale);
+                const float2 v = make_float2(re[e] * un, im[e] * un);
+                float2 x = cmac(v, f, B), t;
+                if constexpr (ST == 1) {
+                  zr[e] = v.x; zi[e] = v.y;
+                  t = cmul(g.c.d1, v);
+                } else {
+                  x = cmul(g.c.r, x);
+                  t = cmac(cmac(B, g.c.g, make_float2(zr[e], zi[e])), g.c.e1, v);
+                }
+                xr[e] = x.x; xi[e] = x.y;
+                re[e] = t.x; im[e] = t.y;
               }
-              f4v* p = z_at(q, a, c);
-              p[0] = zr;
-              p[1] = zi;
+              if constexpr (ST == 1) { p[0] = zr; p[1] = zi; }
+              put_rows(image(q, a, c), xr, xi, sc);
             }
           }
       }
-      if constexpr (ST == 1) {
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-          for (int c = 0; c < 2; c++) { acc[q].re[a][c] = m[a][c][0]; acc[q].im[a][c] = m[a][c][1]; }
+      if constexpr (kB)
         if (NS < 4 && q + 1 < NS) ask(q + 1);
-      }
-      if constexpr (ST == 2)
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-          for (int c = 0; c < 2; c++) {
-            const f4v* p = z_at(q, a, c);
-            acc[q].re[a][c] = p[0];
-            acc[q].im[a][c] = p[1];
-          }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  next_operand(std::integral_constant<int, 0>{});
   product(std::integral_constant<int, 0>{});
   next_operand(std::integral_constant<int, 1>{});
   product(std::integral_constant<int, 1>{});
@@ -524,9 +464,9 @@ bool sym_onchip(int n) { return n <= 224; }
 // One, two, three and four-tile matrices: several workgroups per CU share the matrix cores; from
 // five tiles on one workgroup of eight waves fills the CU.
 void launch_expm_sym(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
-                     float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c) {
+                     const float* bmax, float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c) {
   if (nb <= 0) return;
-  const ExpmArgs a{A, sq, bexp, nb, F, (float*)Q, (_Float16*)spill, c};
+  const ExpmArgs a{A, sq, bexp, bmax, nb, F, (float*)Q, (_Float16*)spill, c};
   switch (n / 32) {
     case 1: return expm_case<1, 1, 1, 1, 3, 12>(s, nb, cus, a);
     case 2: return expm_case<2, 1, 3, 3, 2, 6>(s, nb, cus, a);

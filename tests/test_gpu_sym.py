@@ -50,3 +50,29 @@ def test_symmetric_exponential_sizes(crystal, weak):
         print(f"{crystal} {weak}: npad {p}: {rel[pad[pick] == p].max():.1e}", flush=True)
     assert np.isfinite(got).all() and rel.max() < 1e-4
     assert (np.abs(got - full) / np.abs(ref)).max() < 2e-4
+
+
+@pytest.mark.parametrize("crystal,ekev,weak,nz,dz", [("fe", 26.8, 17.2, 30, 2.0), ("ni", 26.87, 67.6, 24, 0.5), ("fe", 16.41, 13.5, 53, 1.0),
+                                                     ("fe", 20.0, 4.0, 50, 0.5), ("ni", 13.37, 6.5, 46, 1.0)])
+def test_few_beams_against_fp64(crystal, ekev, weak, nz, dz):
+    """Sets of few beams, where the matrix's 1-norm is nearly its spectral radius and the polynomial's truncation is
+    seen in full. Bound: twice what a degree-8 polynomial at the norm 5/4 costs by truncation there (1e-7 to 3e-7), with the
+    same again for the 22-bit operands and the FP32 sums."""
+    from ctemsoft_amd import ebsd, workloads, xtal
+    wl = workloads.get({"fe": "fe_c1", "ni": "ni_c0"}[crystal])
+    st, _ = xtal.native_setup(wl.xtal, ekev, wl.dmin, (weak, 2.0 * weak, 0.05))
+    npx, npy = ebsd.lambert_dims(25, st.usehex)
+    _, k, kn = ebsd.kvectors(npx, npy, st.isym, st.usehex, st.dsm, st.mlambda)
+    z = dz * np.arange(1, nz + 1)
+    lam = (np.exp(-z / 15.0) / np.exp(-z / 15.0).sum()).astype(np.float32)
+    ctx = ebsd.Context(0)
+    ctx.upload_crystal(st)
+    p = ctx.plan(k, kn, lam, dz, float(max(1, int(nz * dz))))
+    ns, _ = p.select()
+    p.run("fp64")
+    ref = p.dots().copy()
+    p.run("mixed")
+    err = np.linalg.norm(p.dots() - ref) / np.linalg.norm(ref)
+    ctx.close()
+    print(f"{crystal} {ekev} kV {weak}: {ns.min()}..{ns.max()} beams, {len(kn)} directions: {err:.2e}", flush=True)
+    assert err < 1.2e-6
