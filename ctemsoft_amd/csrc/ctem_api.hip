@@ -1149,7 +1149,12 @@ int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W
   for (int b = 0; b < nb; b++) fl += (3 + h_sq[b]) * pflops(b);
   GemmTimer t{tp, s};
   t.begin();
-  launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), mx(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
+  if (sym_few(npad, nb)) {
+    float2* const work[4] = {W32 + per * nb, W32 + 2 * per * nb, W32 + 4 * per * nb, W32 + 5 * per * nb};
+    launch_sym_few(s, npad, nb, W32, d_sq, ex(0), mx(0), Ff, work, mx(1), smax, coef);
+  } else {
+    launch_expm_sym(s, npad, nb, W32, d_sq, ex(0), mx(0), Ff, W32 + per * nb, S(2), depth_grid, coef);
+  }
   t.end();
   HIPCHK(hipGetLastError());
   if (tp) { tp->f_gemm += fl; tp->n_gemm++; }

@@ -337,6 +337,11 @@ bool sym_onchip(int n);
 // squaring counts, exponents and maxima of B = A 2^-sq, one launch. Q, spill: work space, n n 8 bytes per matrix.
 void launch_expm_sym(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
                      const float* bmax, float2* F, float2* Q, uint16_t* spill, int32_t cus, const SymCoef& c);
+// the same for a few matrices of six or seven tiles a side, a product per launch (smax: the largest count): work holds
+// four buffers of nb n n entries, maxima 3 nb zeros
+bool sym_few(int n, int nb);
+void launch_sym_few(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
+                    const float* bmax, float2* F, float2* const work[4], float* maxima, int32_t smax, const SymCoef& c);
 // zero `bytes` bytes (a multiple of 4) of device memory with a kernel (no memset node, so that
 // the sequence can be captured into a graph)
 void launch_fill_zero(hipStream_t s, void* p, size_t bytes);

@@ -113,37 +113,32 @@ struct Reader {
 // one tile's accumulators: 16 x 16 subtiles [a][c], lane rows 4 (lane >> 4) + e, column lane & 15
 struct Acc {
   f4v re[2][2], im[2][2];
-  __device__ __forceinline__ void zero() {
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int c = 0; c < 2; c++) { re[a][c] = (f4v){0, 0, 0, 0}; im[a][c] = (f4v){0, 0, 0, 0}; }
-  }
-  // += A B^T over 32 k for column block c. The twelve products go into fresh sums, added to the
-  // accumulators by rounded FP32 additions: the matrix cores' own accumulation does not round to nearest, and
-  // over a whole product its one-sided errors add up (intensities of fcc Ni 9.2e-7 from the 64-bit ones with
-  // the products accumulated in place). The imaginary planes of B are negated for the last terms,
-  // -Im A Im B. Smallest terms first.
-  __device__ __forceinline__ void mma(const h8v (&x)[2][4], h8v (&y)[4], int c) {
-    f4v r[2], i[2];
+};
+
+// re, im += A B^T over 32 k, for the two row blocks of A and one column block. The twelve products go into fresh sums, added
+// to the accumulators by rounded FP32 additions: the matrix cores' own accumulation does not round to nearest, and
+// over a whole product its one-sided errors add up (intensities of fcc Ni 9.2e-7 from the 64-bit ones with
+// the products accumulated in place). The imaginary planes of B are negated for the last terms,
+// -Im A Im B. Smallest terms first.
+__device__ __forceinline__ void mma(const h8v (&x)[2][4], h8v (&y)[4], f4v& re0, f4v& re1, f4v& im0, f4v& im1) {
+  f4v r[2], i[2];
 #define MM(acc, a, u, v) acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[a][u], y[v], acc[a], 0, 0, 0)
 #define MM4(u, v, w, z) MM(r, 0, u, v); MM(r, 1, u, v); MM(i, 0, w, z); MM(i, 1, w, z)
-    r[0] = r[1] = i[0] = i[1] = (f4v){0, 0, 0, 0};
-    MM4(1, 0, 1, 2);
-    MM4(0, 1, 0, 3);
-    MM(i, 0, 3, 0); MM(i, 1, 3, 0); MM(i, 0, 2, 1); MM(i, 1, 2, 1);
-    MM4(0, 0, 0, 2);
+  r[0] = r[1] = i[0] = i[1] = (f4v){0, 0, 0, 0};
+  MM4(1, 0, 1, 2);
+  MM4(0, 1, 0, 3);
+  MM(i, 0, 3, 0); MM(i, 1, 3, 0); MM(i, 0, 2, 1); MM(i, 1, 2, 1);
+  MM4(0, 0, 0, 2);
 #pragma unroll
-    for (int p = 2; p < 4; p++) y[p] = __builtin_bit_cast(h8v, __builtin_bit_cast(u4v, y[p]) ^ 0x80008000u);
-    MM4(3, 2, 2, 0);
-    MM(r, 0, 2, 3); MM(r, 1, 2, 3);
-    MM(r, 0, 2, 2); MM(r, 1, 2, 2);
+  for (int p = 2; p < 4; p++) y[p] = __builtin_bit_cast(h8v, __builtin_bit_cast(u4v, y[p]) ^ 0x80008000u);
+  MM4(3, 2, 2, 0);
+  MM(r, 0, 2, 3); MM(r, 1, 2, 3);
+  MM(r, 0, 2, 2); MM(r, 1, 2, 2);
 #undef MM4
 #undef MM
-#pragma unroll
-    for (int a = 0; a < 2; a++) { re[a][c] += r[a]; im[a][c] += i[a]; }
-  }
-};
+  re0 += r[0]; im0 += i[0];
+  re1 += r[1]; im1 += i[1];
+}
 
 // tile t of the upper triangle in row order (row i: (i, i) .. (i, T - 1))
 __device__ __forceinline__ int row_tile(int t, int T, int& j) {
@@ -158,6 +153,40 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 }
 __device__ __forceinline__ float2 cmac(float2 s, float2 a, float2 b) {  // s + a b
   return make_float2(__builtin_fmaf(-a.y, b.y, __builtin_fmaf(a.x, b.x, s.x)), __builtin_fmaf(a.y, b.x, __builtin_fmaf(a.x, b.y, s.y)));
+}
+
+// Four rows (row ..) of A's column col in tile (i, j), as (re, im) pairs. The table's U(-g) = U(g) holds to about 1e-8
+// only; where the assembly's 64 x 64 tiles give both triangles, their mean is taken (the upper one alone costs
+// corundum's sets of 33-64 beams half of their precision).
+__device__ __forceinline__ void load_a(const float2* A, int n, int i, int j, int row, int col, f4v& m0, f4v& m1) {
+  const f4v* p = (const f4v*)(A + (int64_t)col * n + row);
+  m0 = p[0];
+  m1 = p[1];
+  if (j == i + 1 && !(i & 1)) {
+    const float2* t = A + (int64_t)row * n + col;
+    const float2 t0 = t[0], t1 = t[n], t2 = t[2 * n], t3 = t[3 * n];
+    m0 = 0.5f * (m0 + (f4v){t0.x, t0.y, t1.x, t1.y});
+    m1 = 0.5f * (m1 + (f4v){t2.x, t2.y, t3.x, t3.y});
+  }
+}
+
+// exponent of the operand of step ST (1, 2: a bound of the sum) from the exact maximum of the accumulators before it
+template <int ST>
+__device__ __forceinline__ int operand_exp(const SymCoef& k, float vmax, float bmax) {
+  auto mag = [](float2 v) __attribute__((always_inline)) { return fabsf(v.x) + fabsf(v.y); };
+  if (ST == 1) vmax = __builtin_fmaf(mag(k.c), bmax, vmax);
+  if (ST == 2) vmax = mag(k.r) * __builtin_fmaf(mag(k.d2), bmax, vmax);
+  return f16_scale_exp(vmax);
+}
+
+// F's tile (i, j): four rows of one column, and mirrored off the diagonal
+__device__ __forceinline__ void put_f(float2* F, int n, int i, int j, int row, int col, const f4v& vr, const f4v& vi) {
+  f4v* p = (f4v*)(F + (int64_t)col * n + row);
+  p[0] = (f4v){vr[0], vi[0], vr[1], vi[1]};
+  p[1] = (f4v){vr[2], vi[2], vr[3], vi[3]};
+  if (i != j)
+#pragma unroll
+    for (int e = 0; e < 4; e++) F[(int64_t)(row + e) * n + col] = make_float2(vr[e], vi[e]);
 }
 
 // ---- the whole exponential on chip ------------------------------------------------------------
@@ -272,9 +301,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
           }
           const _Float16* t = row_at(k, sj[q]);
           rd.read(t, 0, sj[q] < k, y[0]);
-          acc[q].mma(x, y[0], 0);
+          mma(x, y[0], acc[q].re[0][0], acc[q].re[1][0], acc[q].im[0][0], acc[q].im[1][0]);
           rd.read(t, 1, sj[q] < k, y[1]);
-          acc[q].mma(x, y[1], 1);
+          mma(x, y[1], acc[q].re[0][1], acc[q].re[1][1], acc[q].im[0][1], acc[q].im[1][1]);
         }
     }
   };
@@ -288,20 +317,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const int l15 = ln & 15, g4 = ln >> 4;
-    // four rows of A, (re, im) pairs. The table's U(-g) = U(g) holds to about 1e-8 only; where the assembly's 64 x 64
-    // tiles give both triangles, their mean is taken (the upper one alone costs corundum's sets of 33-64 beams
-    // half of their precision)
     auto load_b = [&](int q, int a, int c, f4v& m0, f4v& m1) __attribute__((always_inline)) {
-      const int row = 32 * si[q] + 16 * a + 4 * g4, col = 32 * sj[q] + 16 * c + l15;
-      const f4v* p = (const f4v*)(A + (int64_t)col * n + row);
-      m0 = p[0];
-      m1 = p[1];
-      if (T > 1 && sj[q] == si[q] + 1 && !(si[q] & 1)) {
-        const float2* t = A + (int64_t)row * n + col;
-        const float2 t0 = t[0], t1 = t[n], t2 = t[2 * n], t3 = t[3 * n];
-        m0 = 0.5f * (m0 + (f4v){t0.x, t0.y, t1.x, t1.y});
-        m1 = 0.5f * (m1 + (f4v){t2.x, t2.y, t3.x, t3.y});
-      }
+      load_a(A, n, si[q], sj[q], 32 * si[q] + 16 * a + 4 * g4, 32 * sj[q] + 16 * c + l15, m0, m1);
     };
     auto z_at = [&](int q, int a, int c) __attribute__((always_inline)) {
       return (f4v*)(Q + (int64_t)min(t0 + q, N - 1) * 2048) + ln * 2 + (2 * a + c) * 128;
@@ -364,12 +381,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
     vmax = red[0];
 #pragma unroll
     for (int w = 1; w < NW; w++) vmax = fmaxf(vmax, red[w]);
-    vmax *= un;
-    auto mag = [](float2 v) __attribute__((always_inline)) { return fabsf(v.x) + fabsf(v.y); };
     const float2 f = ST == 1 ? g.c.c : g.c.d2;
-    if constexpr (ST == 1) vmax += mag(f) * g.bmax[b];
-    if constexpr (ST == 2) vmax = mag(g.c.r) * (vmax + mag(f) * g.bmax[b]);
-    ex = f16_scale_exp(vmax);
+    ex = operand_exp<ST>(g.c, vmax * un, kB ? g.bmax[b] : 0.0f);
     const float sc = ldexpf(kB ? 1.0f : un, ex);
 #pragma unroll
     for (int q = 0; q < NS; q++) {
@@ -434,13 +447,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(EU, EU)
 #pragma unroll
         for (int c = 0; c < 2; c++) {
           const int row = 32 * i + 16 * a + 4 * g4, col = 32 * j + 16 * c + l15;
-          const f4v vr = acc[q].re[a][c] * un, vi = acc[q].im[a][c] * un;
-          f4v* p = (f4v*)(F + (int64_t)col * n + row);
-          p[0] = (f4v){vr[0], vi[0], vr[1], vi[1]};
-          p[1] = (f4v){vr[2], vi[2], vr[3], vi[3]};
-          if (i != j)
-#pragma unroll
-            for (int e = 0; e < 4; e++) F[(int64_t)(row + e) * n + col] = make_float2(vr[e], vi[e]);
+          put_f(F, n, i, j, row, col, acc[q].re[a][c] * un, acc[q].im[a][c] * un);
         }
     }
   __syncthreads();  // every wave is done with the last operand
@@ -452,6 +459,199 @@ template <int T, int NW, int NS, int NSL, int EU, int kWg>
 void expm_case(hipStream_t s, int nb, int cus, const ExpmArgs& a) {
   hipLaunchKernelGGL((k_expm_sym<T, NW, NS, NSL, EU>), dim3(std::min(nb, kWg * cus)), dim3(NW * 64),
                      NSL * kTile * sizeof(_Float16) + 64, s, a);
+}
+
+// ---- few matrices --------------------------------------------------------------------------------
+
+// The same exponential, bit for bit, a product per launch: a wave takes 32 rows and 16 or 32 columns of a tile, with the
+// operands in FP32 from memory (both triangles, split as they are read) and no exchange but the maximum. For a handful of
+// matrices of six or seven tiles a side, where k_expm_sym leaves most CUs idle: a direction's result may not depend on
+// its batch. Step -1 lays B out (unscaled), 0 to 2 are the polynomial, 3 a squaring. Bound by latency.
+struct FewArgs {
+  const float2* A;
+  const int32_t* sq;
+  const int32_t* bexp;
+  const float* bmax;
+  int32_t n, nb, it;         // it: the squaring's number
+  float2* B;                 // [nb][n n]: what step -1 lays out
+  const float2* X;           // operand in
+  float2* Y;                 // operand out
+  float2* F;                 // out: the result of a matrix's last product
+  float* Q;                  // [nb][N 2048]: B^2, then the terms of step 2
+  const float* max_in;       // [nb]: maximum of the product before, and of this one; `clear` is the next one's
+  float* max_out;
+  float* clear;
+  SymCoef c;
+};
+
+// CB: column blocks of 16 per wave, from c0
+template <int ST, int CB>
+__device__ __forceinline__ void few_step(const FewArgs& g, int b, int t, int c0, int lane) {
+  const int n = g.n, T = n >> 5, l15 = lane & 15, g4 = lane >> 4;
+  const int64_t per = (int64_t)n * n;
+  int j;
+  const int i = row_tile(t, T, j), row0 = 32 * i + 4 * g4, col0 = 32 * j + 16 * c0 + l15;
+  float2* const B = g.B + b * per;
+  if constexpr (ST < 0) {
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int c = 0; c < CB; c++) {
+        const int row = row0 + 16 * a, col = col0 + 16 * c;
+        f4v m0, m1;
+        load_a(g.A + b * per, n, i, j, row, col, m0, m1);
+        put_f(B, n, i, j, row, col, (f4v){m0[0], m0[2], m1[0], m1[2]}, (f4v){m0[1], m0[3], m1[1], m1[3]});
+      }
+    return;
+  } else {
+    const int s = g.sq[b];
+    if (ST == 3 && g.it >= s) return;
+    if (t == 0 && c0 == 0 && lane == 0) g.clear[b] = 0.0f;
+    const float bscale = ldexpf(1.0f, -s);
+    const int ex = ST == 0 ? g.bexp[b] : operand_exp<ST>(g.c, g.max_in[b], g.bmax[b]);
+    const float up = ldexpf(1.0f, 2 * ex), un = ldexpf(1.0f, -2 * ex), sc = ldexpf(ST == 0 ? bscale : 1.0f, ex);
+    const float2* X = (ST == 0 ? B : g.X + b * per);
+    auto z_at = [&](int a, int c) __attribute__((always_inline)) {
+      return (f4v*)(g.Q + b * (per * 2)) + ((int64_t)t * 512 + lane * 2 + (2 * a + c0 + c) * 128);
+    };
+    // (re, im) of four rows of one column of a matrix
+    auto load4 = [&](const float2* M, int a, int c, f4v& r, f4v& im) __attribute__((always_inline)) {
+      const f4v* p = (const f4v*)(M + (int64_t)(col0 + 16 * c) * n + row0 + 16 * a);
+      const f4v m0 = p[0], m1 = p[1];
+      r = (f4v){m0[0], m0[2], m1[0], m1[2]};
+      im = (f4v){m0[1], m0[3], m1[1], m1[3]};
+    };
+    f4v re[CB][2], im[CB][2];
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        f4v &r = re[c][a], &m = im[c][a];
+        r = m = (f4v){0, 0, 0, 0};
+        if constexpr (ST == 1 || ST == 2) {
+          const f4v* z = z_at(a, c);
+          const f4v zr = z[0], zi = z[1];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float2 v = ST == 1 ? cmul(g.c.d1, make_float2(zr[e], zi[e])) : make_float2(zr[e], zi[e]);
+            r[e] = v.x * up;
+            m[e] = v.y * up;
+          }
+        }
+        if constexpr (ST == 3) {
+          load4(X, a, c, r, m);
+          r *= 2.0f * up;
+          m *= 2.0f * up;
+        }
+      }
+    // eight k of a row or column, split
+    auto split8 = [&](const float2 (&v)[8], h8v (&o)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        o[0][e] = (_Float16)(v[e].x * sc);
+        o[2][e] = (_Float16)(v[e].y * sc);
+        o[1][e] = (_Float16)__builtin_fmaf(v[e].x, sc, -(float)o[0][e]);
+        o[3][e] = (_Float16)__builtin_fmaf(v[e].y, sc, -(float)o[2][e]);
+      }
+    };
+    auto column = [&](int q, int k, float2 (&v)[8]) __attribute__((always_inline)) {  // rows k .. of column q
+      const f4v* p = (const f4v*)(X + (int64_t)q * n + k);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const f4v u = p[e];
+        v[2 * e] = make_float2(u[0], u[1]);
+        v[2 * e + 1] = make_float2(u[2], u[3]);
+      }
+    };
+#pragma unroll 1
+    for (int k = 0; k < T; k++) {
+      const int k0 = 32 * k + 8 * g4;
+      float2 vx[2][8], vy[CB][8];
+#pragma unroll
+      for (int c = 0; c < CB; c++) column(col0 + 16 * c, k0, vy[c]);
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        const int r = 32 * i + 16 * a + l15;
+        if (i == k) {  // the diagonal tile: row r itself
+#pragma unroll
+          for (int e = 0; e < 8; e++) vx[a][e] = X[(int64_t)(k0 + e) * n + r];
+        } else {
+          column(r, k0, vx[a]);
+        }
+      }
+      h8v x[2][4], y[4];
+      split8(vx[0], x[0]);
+      split8(vx[1], x[1]);
+#pragma unroll
+      for (int c = 0; c < CB; c++) {
+        split8(vy[c], y);
+        mma(x, y, re[c][0], re[c][1], im[c][0], im[c][1]);
+      }
+    }
+    float vmax = 0.0f;
+    const bool last = (ST == 2 && s == 0) || (ST == 3 && g.it + 1 == s);
+    float2* const out = (last ? g.F : g.Y) + b * per;
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        const f4v r = re[c][a] * un, m = im[c][a] * un;
+        const int row = row0 + 16 * a, col = col0 + 16 * c;
+#pragma unroll
+        for (int e = 0; e < 4; e++) vmax = fmaxf(vmax, fmaxf(fabsf(r[e]), fabsf(m[e])));
+        if constexpr (ST < 2) {
+          f4v br, bi, zr, zi, xr, xi;
+          load4(B, a, c, br, bi);
+          f4v* z = z_at(a, c);
+          if constexpr (ST == 1) { zr = z[0]; zi = z[1]; }
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float2 bv = make_float2(br[e] * bscale, bi[e] * bscale), v = make_float2(r[e], m[e]);
+            float2 x = cmac(v, ST == 0 ? g.c.c : g.c.d2, bv), w = v;
+            if constexpr (ST == 1) {
+              x = cmul(g.c.r, x);
+              w = cmac(cmac(bv, g.c.g, make_float2(zr[e], zi[e])), g.c.e1, v);
+            }
+            zr[e] = w.x; zi[e] = w.y;
+            xr[e] = x.x; xi[e] = x.y;
+          }
+          z[0] = zr;
+          z[1] = zi;
+          put_f(out, n, i, j, row, col, xr, xi);
+        } else {
+          put_f(out, n, i, j, row, col, r, m);
+        }
+      }
+    if (!last) wave_max_to(vmax, g.max_out + b);
+  }
+}
+
+template <int ST, int CB>
+__global__ __launch_bounds__(64) void k_sym_few(FewArgs g) {
+  const int T = g.n >> 5, per = T * (T + 1) / CB;  // waves of a matrix, which keep to one XCD's L2
+  const int w = xcd_logical_block(blockIdx.x, gridDim.x), b = w / per, u = w % per;
+  few_step<ST, CB>(g, b, CB == 2 ? u : u >> 1, CB == 2 ? 0 : u & 1, threadIdx.x);
+}
+
+template <int CB>
+void few_steps(hipStream_t s, FewArgs g, float2* const work[4], float* maxima, int smax) {
+  const int T = g.n / 32;
+  const dim3 grid(g.nb * T * (T + 1) / CB), blk(64);
+  g.B = work[0];
+  g.Q = (float*)work[1];
+  hipLaunchKernelGGL((k_sym_few<-1, CB>), grid, blk, 0, s, g);
+  for (int i = 0; i < 3 + smax; i++) {
+    g.X = work[2 + (i & 1)];
+    g.Y = work[2 + ((i + 1) & 1)];
+    g.max_in = maxima + (i % 3) * g.nb;
+    g.max_out = maxima + ((i + 1) % 3) * g.nb;
+    g.clear = maxima + ((i + 2) % 3) * g.nb;
+    g.it = i - 3;
+    if (i == 0) hipLaunchKernelGGL((k_sym_few<0, CB>), grid, blk, 0, s, g);
+    else if (i == 1) hipLaunchKernelGGL((k_sym_few<1, CB>), grid, blk, 0, s, g);
+    else if (i == 2) hipLaunchKernelGGL((k_sym_few<2, CB>), grid, blk, 0, s, g);
+    else hipLaunchKernelGGL((k_sym_few<3, CB>), grid, blk, 0, s, g);
+  }
 }
 
 }  // namespace
@@ -476,6 +676,19 @@ void launch_expm_sym(hipStream_t s, int32_t n, int32_t nb, const float2* A, cons
     case 6: return expm_case<6, 8, 3, 19, 2, 1>(s, nb, cus, a);
     case 7: return expm_case<7, 8, 4, 19, 2, 1>(s, nb, cus, a);
   }
+}
+
+// One MI355X, a run of bcc Fe with 20 depths [us], this / k_expm_sym / k_sgemm's chain. 161-187 beams: 1 direction
+// 258 / 341 / 322, 48 directions 341 / 351 / 391, 56 365 / 351 / 393. 193-211 beams: 1 direction 292 / 467 / 357, 32 380 / 478 / 429,
+// 56 478 / 487 / 472, 64 506 / 488 / 485. Smaller matrices are no slower in one launch than in k_sgemm's chain.
+bool sym_few(int n, int nb) { return n > 160 && n <= 224 && nb <= n / 4; }
+
+void launch_sym_few(hipStream_t s, int32_t n, int32_t nb, const float2* A, const int32_t* sq, const int32_t* bexp,
+                    const float* bmax, float2* F, float2* const work[4], float* maxima, int32_t smax, const SymCoef& c) {
+  const FewArgs g{A, sq, bexp, bmax, n, nb, 0, nullptr, nullptr, nullptr, F, nullptr, nullptr, nullptr, nullptr, c};
+  // half as wide while there are fewer waves than SIMDs
+  if (nb <= 12) few_steps<1>(s, g, work, maxima, smax);
+  else few_steps<2>(s, g, work, maxima, smax);
 }
 
 }  // namespace ctem

@@ -76,3 +76,38 @@ def test_few_beams_against_fp64(crystal, ekev, weak, nz, dz):
     ctx.close()
     print(f"{crystal} {ekev} kV {weak}: {ns.min()}..{ns.max()} beams, {len(kn)} directions: {err:.2e}", flush=True)
     assert err < 1.2e-6
+
+
+@pytest.mark.parametrize("weak,npad,count", [(4.0, 32, 3200), (60.0, 64, 1700), (100.0, 96, 700), (140.0, 128, 700), (190.0, 160, 400),
+                                             (250.0, 192, 400), (320.0, 224, 400)])
+def test_batch_sizes_bitwise(weak, npad, count):
+    """More matrices than workgroups (each then walks several, with the same LDS, spill and work buffers) against the same
+    directions alone and in small batches, on both sides of where the largest sizes change from a product per launch
+    (one and two column blocks a wave) to one launch: the same bits."""
+    from ctemsoft_amd import ebsd, workloads, xtal
+    wl = workloads.get("fe_c1")
+    st, _ = xtal.native_setup(wl.xtal, wl.ekev, wl.dmin, (weak, 2.0 * weak, 0.05))
+    npx, npy = ebsd.lambert_dims(40, st.usehex)
+    _, k, kn = ebsd.kvectors(npx, npy, st.isym, st.usehex, st.dsm, st.mlambda)
+    lam = np.exp(-np.arange(1, 6) / 8.0).astype(np.float32)
+    ctx = ebsd.Context(0)
+    ctx.upload_crystal(st)
+
+    def dots(i):
+        p = ctx.plan(k[i], kn[i], lam, 1.0, 5.0)
+        ns, _ = p.select()
+        p.run("mixed")
+        d = p.dots().copy()
+        p.close()
+        return ns, d
+    ns, _ = dots(np.arange(len(kn)))
+    idx = np.flatnonzero(np.maximum(32, (ns + 31) // 32 * 32) == npad)
+    assert len(idx) > 70, (npad, ns.min(), ns.max())
+    big = np.resize(idx, count)
+    _, ref = dots(big)
+    assert np.isfinite(ref).all()
+    again = ref[len(idx):2 * len(idx)]
+    assert np.array_equal(again, ref[:len(again)])
+    for n in (1, 3, 12, 13, npad // 4, npad // 4 + 1):
+        assert np.array_equal(dots(idx[:n])[1], ref[:n]), n
+    ctx.close()
