@@ -457,8 +457,9 @@ __device__ __forceinline__ void zg_run(const ZGemm& g, const ZgTile& t, int b, i
   if (nk) issue(0, 0);
   for (int c = 0; c < nk; c++) {
     const int z = c & 1;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // chunk c has arrived, and every wave is done with the other buffer
+    // chunk c has arrived, and every wave's reads of the other buffer have returned
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (c + 1 < nk) issue(c + 1, z ^ 1);
     const int kc = 8 * (c >= nk1 ? c - nk1 : c);
