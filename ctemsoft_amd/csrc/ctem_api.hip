@@ -2091,12 +2091,25 @@ extern "C" int32_t ctem_plan_scatter(ctem_plan* p, const int32_t* ij, int32_t np
   return CTEM_OK;
 }
 
+// The products of a channeling plan's one-launch directions, kept behind its intensities: int32 per direction, 0 for others
+static size_t ecp_nprod_at(const ctem_plan* p) { return sizeof(float) * (size_t)p->ecp_nt * std::max(p->numk, 1); }
+
 extern "C" int32_t ctem_plan_timing(ctem_plan* p, double* total_ms, double* gemm_ms, double* gemm_flops,
                                     int32_t* gemm_launches) {
   if (!p || !p->ran) return fail(CTEM_E_STATE, "ctem_plan_timing: run the plan first");
   if (total_ms) *total_ms = p->t_total;
   if (gemm_ms) *gemm_ms = p->t_gemm;
-  if (gemm_flops) *gemm_flops = p->f_gemm;
+  if (gemm_flops) {
+    double f = 0.0;
+    if (p->ecp_mode >= 0 && p->numk > 0) {
+      std::vector<int32_t> np(p->numk);
+      HIPCHK(hipMemcpy(np.data(), (char*)p->ecp_sr.p + ecp_nprod_at(p), 4 * np.size(), hipMemcpyDeviceToHost));
+      const double solve = p->ecp_mode == CTEM_ECP_SCATMAT ? 32.0 / 3.0 : 0.0;
+      for (int i = 0; i < p->numk; i++)
+        if (np[i]) f += (double)p->h_nns[i] * p->h_nns[i] * p->h_nns[i] * (8.0 * np[i] + solve);
+    }
+    *gemm_flops = p->f_gemm + f;
+  }
   if (gemm_launches) *gemm_launches = p->n_gemm;
   return CTEM_OK;
 }
@@ -2338,7 +2351,7 @@ static void build_slut_ecp(const Crystal& cr, const float* occ, std::vector<doub
 // A z0, overwritten with the scaled B); W holds 5 nb npad^2 entries of work space, d_q and d_j nb
 // integers each. Returns the slice of W that holds E.
 static double2* pade_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double2* A, double2* W, int32_t* d_q,
-                          int32_t* d_j, int32_t* d_err, int32_t& rc_out) {
+                          int32_t* d_j, int32_t* d_err, const std::vector<int>& h_n, int32_t& rc_out) {
   rc_out = CTEM_OK;
   const int64_t per = (int64_t)npad * npad;
   double2* C0 = W;
@@ -2357,6 +2370,7 @@ static double2* pade_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double
     t.begin();
     launch_zgemm(s, g);
     t.end();
+    tp->n_gemm++;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { rc_out = fail(CTEM_E_HIP, "Pade product: %s", hipGetErrorString(e)); return false; }
     return true;
@@ -2369,12 +2383,16 @@ static double2* pade_fp64(ctem_plan* tp, hipStream_t s, int npad, int nb, double
     if (icnt < 4 && !prod(cb[icnt & 1], cb[(icnt - 1) & 1], A, d_q, icnt - 1)) return nullptr;
   }
   launch_zsolve(s, npad, nb, D, N, d_err);
-  std::vector<int32_t> hj(nb);
+  std::vector<int32_t> hj(nb), hq(nb);  // hq: products of the sums
   hipError_t e = hipMemcpyAsync(hj.data(), d_j, 4 * (size_t)nb, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(hq.data(), d_q, 4 * (size_t)nb, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) { rc_out = fail(CTEM_E_HIP, "Pade squaring counts: %s", hipGetErrorString(e)); return nullptr; }
   int jmax = 0;
-  for (int b = 0; b < nb; b++) jmax = std::max(jmax, hj[b]);
+  for (int b = 0; b < nb; b++) {
+    jmax = std::max(jmax, hj[b]);
+    tp->f_gemm += 8.0 * h_n[b] * h_n[b] * h_n[b] * (hq[b] + hj[b]);
+  }
   double2* buf[2] = {N, T};
   for (int i = 0; i < jmax; i++)
     if (!prod(buf[(i + 1) & 1], buf[i & 1], buf[i & 1], d_j, i)) return nullptr;
@@ -2442,7 +2460,7 @@ extern "C" int32_t ctem_ecp_plan_create(ctem_ctx* c, int32_t numk, const double*
   if ((rc = upload(p->fn, prm->fn, 3, s)) || (rc = upload(p->ecp_slut, slut.data(), slut.size(), s)) ||
       (rc = upload(p->ecp_thick, thick.data(), thick.size(), s)) ||
       (numt > 0 && (rc = upload(p->ecp_store, store.data(), store.size(), s))) ||
-      (rc = p->ecp_sr.ensure(sizeof(float) * (size_t)nt * std::max(numk, 1)))) {
+      (rc = p->ecp_sr.ensure(ecp_nprod_at(p) + 4 * (size_t)std::max(numk, 1)))) {
     ctem_plan_destroy(p);
     *out = nullptr;
     return rc;
@@ -2508,7 +2526,8 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
   reset_timing(p);
   HIPCHK(hipEventRecord(c->ev[0], s));
   launch_fill_zero(s, p->err.p, 4);
-  launch_fill_zero(s, p->ecp_sr.p, sizeof(float) * (size_t)nt * std::max(p->numk, 1));
+  launch_fill_zero(s, p->ecp_sr.p, ecp_nprod_at(p) + 4 * (size_t)std::max(p->numk, 1));
+  int32_t* nprod = (int32_t*)((char*)p->ecp_sr.p + ecp_nprod_at(p));
   BeamView V{p->nns.as<int32_t>(), p->nnw.as<int32_t>(), p->soff.as<int64_t>(), p->woff.as<int64_t>(),
              p->sidx.as<int32_t>(), p->ssg.as<float>(), p->widx.as<int32_t>(), p->wsg.as<float>()};
   DevRefl R = p->cr->refl();
@@ -2528,15 +2547,18 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
       std::vector<int32_t> hsq;
       if (ecp_small(npad)) {
         double2* A = c->w.A.as<double2>();
-        if (bloch) {
-          launch_assemble(s, B, V, R, L, p->kn.as<double>(), p->cr->mlambda, p->cr->dynupz, 1.0, A);
+        if (bloch) launch_assemble(s, B, V, R, L, p->kn.as<double>(), p->cr->mlambda, p->cr->dynupz, 1.0, A);
+        else launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, A);
+        GemmTimer t{p, s};
+        t.begin();
+        if (bloch)
           launch_ecp_bloch_small(s, B, V, R, LE, A, (double)p->ecp_t0, (double)p->ecp_dt, nt, p->ecp_thick.as<float>(),
-                                 p->ecp_nat, p->numk, p->err.as<int32_t>(), p->ecp_sr.as<float>());
-        } else {
-          launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, A);
+                                 p->ecp_nat, p->numk, p->err.as<int32_t>(), p->ecp_sr.as<float>(), nprod);
+        else
           launch_ecp_scat_small(s, B, V, R, LE, A, numt, p->ecp_store.as<int32_t>(), p->ecp_nat, p->numk,
-                                p->err.as<int32_t>(), p->ecp_sr.as<float>());
-        }
+                                p->err.as<int32_t>(), p->ecp_sr.as<float>(), nprod);
+        t.end();
+        p->n_gemm++;
         HIPCHK(hipGetLastError());
       } else if (!bloch) {
         for (int b = 0; b < nb; b++) hn.push_back(p->h_nns[kv.second[c0 + b]]);
@@ -2544,7 +2566,7 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
         launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, c->w.A.as<double2>());
         HIPCHK(hipGetLastError());
         double2* E = pade_fp64(p, s, npad, nb, c->w.A.as<double2>(), c->w.W.as<double2>(), c->w.sq.as<int32_t>(),
-                               c->w.sq.as<int32_t>() + nb, p->err.as<int32_t>(), rc);
+                               c->w.sq.as<int32_t>() + nb, p->err.as<int32_t>(), hn, rc);
         if (!E) return rc;
         const int64_t spsi = (int64_t)npad * numt;
         launch_depth(s, npad, nb, numt, E, 0, 0, c->w.Psi.as<double2>(), spsi, c->cu_count);

@@ -148,7 +148,7 @@ template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4 : 1, NT == 1 ? 4 : 1)))
 void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* __restrict__ A1, double t0, double dt,
                        int nt, const float* __restrict__ thick, double nat, int numk, int32_t* __restrict__ err,
-                       float* __restrict__ sr) {
+                       float* __restrict__ sr, int32_t* __restrict__ nprod) {
   typedef Wg<NT> W;
   constexpr int NP = W::NP, LD = W::LD;
   extern __shared__ double2 lds[];
@@ -178,6 +178,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
   });
 
   // E(t) into P0 and M(t) into P1
+  int products = 0;
   auto propagators = [&](double t) __attribute__((always_inline)) {
     int s = 0;
     double x = nrm * t;
@@ -188,6 +189,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
       if (x > kThetaSmall && tid == 0) atomicOr(err, 4);
     }
     const double h = ldexp(t, -s);
+    products += kDegM + 5 + 3 * s;
     typename W::Acc er, ei, mr, mi, cr, ci;
     __syncthreads();
     for (int e = tid; e < NP * NP; e += 256) {
@@ -276,8 +278,9 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
   double run = P1[0].x;
   if (tid < NP) psi[tid] = P0[tid];
   if (tid == 0) sr[dir] = (float)(run / (double)thick[0] / nat);
+  if (nt >= 2 && dt != t0) propagators(dt);
+  if (tid == 0) nprod[dir] = products;
   if (nt < 2) return;
-  if (dt != t0) propagators(dt);
   __syncthreads();
   for (int it = 1; it < nt; it++) {
     const double2* u = psi + ((it - 1) & 1) * NP;
@@ -300,7 +303,7 @@ template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NT == 1 ? 4 : 1)))
 void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* __restrict__ A1, int nz,
                       const int32_t* __restrict__ store, double nat, int numk, int32_t* __restrict__ err,
-                      float* __restrict__ sr) {
+                      float* __restrict__ sr, int32_t* __restrict__ nprod) {
   typedef Wg<NT> W;
   constexpr int NP = W::NP, LD = W::LD;
   extern __shared__ double2 lds[];
@@ -332,6 +335,7 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
   const int q = ilev == 1 ? 2 : ilev == 2 ? 3 : 4;
   const int j2 = ilev <= 2 ? 0 : ilev == 3 ? 1 : ilev == 4 ? 5 : ilev == 5 ? 8 : 11;
   const double sc = ldexp(1.0, -j2);
+  if (tid == 0) nprod[dir] = q - 1 + j2;
   // N = sum pref_i B^i, D = sum (-1)^i pref_i B^i with the reference's running product pref
   w.each([&](int i, int j, int e, int r, int c) {
     double2 v = P0[c * LD + r];
@@ -478,29 +482,29 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
 
 }  // namespace
 
-// two matrices and the exchange buffers in LDS: 35 KB at 32 beams, 143 KB at 64
+// two matrices and the exchange buffers in LDS: 35 KB at 32 beams, 136 KB at 64
 bool ecp_small(int npad) { return npad <= 64; }
 
 void launch_ecp_bloch_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                             const double2* A1, double t0, double dt, int32_t nt, const float* thick, double nat,
-                            int32_t numk, int32_t* err, float* sr) {
+                            int32_t numk, int32_t* err, float* sr, int32_t* nprod) {
   if (B.npad == 32)
     hipLaunchKernelGGL(k_ecp_bloch_small<1>, dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
-                       nat, numk, err, sr);
+                       nat, numk, err, sr, nprod);
   else
     hipLaunchKernelGGL(k_ecp_bloch_small<2>, dim3(B.nb), dim3(256), Wg<2>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
-                       nat, numk, err, sr);
+                       nat, numk, err, sr, nprod);
 }
 
 void launch_ecp_scat_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                            const double2* A1, int32_t nz, const int32_t* store, double nat, int32_t numk, int32_t* err,
-                           float* sr) {
+                           float* sr, int32_t* nprod) {
   if (B.npad == 32)
     hipLaunchKernelGGL(k_ecp_scat_small<1>, dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, nz, store, nat, numk,
-                       err, sr);
+                       err, sr, nprod);
   else
     hipLaunchKernelGGL(k_ecp_scat_small<2>, dim3(B.nb), dim3(256), Wg<2>::lds(), s, B, V, R, L, A1, nz, store, nat, numk,
-                       err, sr);
+                       err, sr, nprod);
 }
 
 }  // namespace ctem

@@ -45,3 +45,36 @@ def test_small_sets(key, weak, mode, oracle_mod, monkeypatch):
         want, *_ = oracle_mod.ecp_direction(cr, geo["k"][ik], geo["kn"][ik], geo["dynfn"], mode, thick, 0.5,
                                             exact=mode == "Blochwv")
         assert _ulps(sr[:, ik], want).max() <= 1, (ns[ik], sr[:, ik], want)
+
+
+@pytest.mark.parametrize("mode", ["Blochwv", "ScatMat"])
+@pytest.mark.parametrize("key,weak", [("s1", 30.0), ("s1", 100.0), ("s1", 300.0)])
+def test_timing_counts_the_products(key, weak, mode, monkeypatch):
+    """ctem_plan_timing after a channeling-pattern run, below and above 64 beams: a time, and flops between the
+    fewest and the most products that the mode can take per direction."""
+    import ecp_cases
+    from ctemsoft_amd import ebsd, ecp
+    z = fixture()
+    cut = (weak, 2.0 * weak, 0.05)
+    monkeypatch.setattr(ecp_cases, "setup_params", lambda *a: dict(setup_params(*a), cutoffs=cut))
+    st, _, geo = native_setup(z, key)
+    occ = [s["occ"] for s in setup_params(z, key)["xtal"]["sites"]]
+    ctx = ebsd.Context(0)
+    try:
+        ctx.upload_crystal(st)
+        p = ecp.EcpPlan(ctx, geo["k"], geo["kn"], mode, 1.5, 2.5, 4, 0.5, geo["dynfn"], occ)
+        ns, _ = p.select()
+        p.run()
+        first = p.timing()
+        p.run()
+        t = p.timing()
+    finally:
+        ctx.close()
+    print(f"{weak} {mode}: {ns.min()}..{ns.max()} beams: {t}", flush=True)
+    n3 = 8.0 * (ns.astype(float) ** 3).sum()
+    assert t["gemm_ms"] > 0 and t["gemm_launches"] > 0 and t["gemm_ms"] <= t["total_ms"]
+    assert t["gemm_flops"] == first["gemm_flops"]
+    few, most = (32, 32 + 6 * 51) if mode == "Blochwv" else (1, 14 + 4)
+    if ns.max() > 64:
+        most *= 8
+    assert few * n3 <= t["gemm_flops"] <= most * n3
