@@ -41,7 +41,9 @@ def master_loss(plan, ij, npx, npy, isym, target, precision="fp64"):
 def master_loss_grad(plan, ij, npx, npy, isym, target, owner=None, precision="fp64"):
     """(loss, dloss/dLUT shaped like the LUT [l][k][h], dloss/dB per site). precision "fp64":
     FP64 forward and reverse pass; "mixed": the loss from the mixed forward and the gradient from
-    the mixed reverse pass (ctem_plan_adjoint_mixed, which reruns the same mixed forward)."""
+    the mixed reverse pass (ctem_plan_adjoint_mixed). Its forward takes full products where the run squares
+    symmetric matrices, so it differentiates at intensities about 1e-6 from those of the loss; with
+    plan.set_symmetry(0) the two forwards are the same."""
     loss, sr = master_loss(plan, ij, npx, npy, isym, target, precision)
     if owner is None:
         owner = pixel_owner(ij, npx, npy, isym)

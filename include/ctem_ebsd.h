@@ -187,8 +187,9 @@ CTEM_API int32_t ctem_plan_dynmat(ctem_plan* plan, int32_t ik, double* dynmat, i
  * direction. */
 CTEM_API int32_t ctem_plan_adjoint(ctem_plan* plan, const double* gdots, double* glut, double* gb);
 /* The same gradient with the mixed forward: psi in the mixed form of ctem_plan_run (for an
- * inversion-symmetric crystal with that form's degree-8 polynomial, within the form's error of
- * ctem_plan_run's intensities), the backward depth recursion in FP64,
+ * inversion-symmetric crystal by full products and a degree-8 polynomial where ctem_plan_run squares
+ * symmetric matrices: the gradient is taken at intensities that differ from that run's by both forms' errors,
+ * about 1e-6 of them; with ctem_plan_set_symmetry(plan, 0) the two forwards are one), the backward depth recursion in FP64,
  * and the Frechet derivative of the exponential on split-FP16 products with FP32 accumulation,
  * its squaring stages recomputed. No counterpart in the reference, as ctem_plan_adjoint. Same
  * arguments and limits. */

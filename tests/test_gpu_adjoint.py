@@ -220,3 +220,43 @@ def test_mixed_adjoint_matches_fp64(ctx, name, symmetry, terms):
     _say(f"{name} symmetry {symmetry} terms {terms}: forward {ed:.2e}, grad LUT {eg:.2e}, grad B {eb:.2e}")
     tol = 2e-3 if terms == 3 else 2e-4
     assert eg <= tol and eb <= tol, (eg, eb)
+
+
+@pytest.mark.parametrize("name,symmetry", [("ni_c0w", 1), ("ni_c0w", 0), ("fe_c1w", 1)])
+def test_mixed_gradient_at_the_runs_intensities(ctx, name, symmetry):
+    """A fit's step: gdots from the residual of run("mixed") against a target, then the mixed gradient, whose own forward
+    may differ from the run's by both forms' errors. Against the FP64 gradient for the same gdots, and the same for the
+    FP64 residual. The mixed intensities are within 2e-6 of the FP64 ones and the derivative's split products add as
+    much; the residuals are 1e-2 of the intensities, so theirs add 2e-4. B's gradient is held to that share of the sum
+    of the directions' absolute contributions."""
+    from ctemsoft_amd import ebsd
+    fx = load_golden(name)
+    rng = np.random.default_rng(33)
+    ks = np.sort(rng.choice(len(fx["kvec"]), 12, replace=False))
+    ctx.upload_crystal(ebsd.Setup.from_fixture(fx))
+    args = (fx["lam"], float(fx["dz"]), float(fx["thick"]))
+    plan = ctx.plan(fx["kvec"][ks], fx["kn"][ks], *args)
+    plan.set_symmetry(symmetry)
+    plan.run("fp64")
+    d64 = plan.dots().copy()
+    target = d64 * (1.0 + 0.01 * rng.standard_normal(d64.shape))
+    plan.run("mixed")
+    dmx = plan.dots().copy()
+    assert (np.abs(dmx - d64) / np.abs(d64)).max() <= 1e-5
+    w = 2.0 * (dmx - target)
+    gmx, bmx = plan.adjoint(w, "mixed")
+    g64, b64 = plan.adjoint(w)
+    gt, bt = plan.adjoint(2.0 * (d64 - target))
+    plan.close()
+    scale = np.zeros_like(b64)
+    for i in range(len(ks)):
+        p = ctx.plan(fx["kvec"][ks[i:i + 1]], fx["kn"][ks[i:i + 1]], *args)
+        p.select()
+        scale += np.abs(p.adjoint(w[i:i + 1])[1])
+        p.close()
+    norm = np.linalg.norm
+    eg, et = norm(gmx - g64) / norm(g64), norm(gmx - gt) / norm(gt)
+    eb = (np.abs(bmx - b64) / scale).max()
+    _say(f"{name} symmetry {symmetry}: LUT {eg:.1e} (against the FP64 residual's {et:.1e}), B {eb:.1e} of its terms")
+    assert eg <= 1e-5 and et <= 1e-3 and eb <= 1e-5
+    assert (np.abs(bmx - bt) / scale).max() <= 1e-3
