@@ -16,9 +16,9 @@ def _ulps(a, b):
 
 
 @pytest.mark.parametrize("mode", ["Blochwv", "ScatMat"])
-@pytest.mark.parametrize("key,weak", [("s1", 2.0), ("s1", 30.0), ("s1", 60.0), ("s1", 100.0), ("s1", 130.0),
-                                      ("s2", 8.0), ("s2", 40.0), ("s2", 60.0)])
-def test_small_sets(key, weak, mode, oracle_mod, monkeypatch):
+@pytest.mark.parametrize("key,weak,sizes", [("s1", 2.0, {32}), ("s1", 30.0, {32}), ("s1", 60.0, {32, 64}), ("s1", 100.0, {64, 96}),
+                                            ("s1", 130.0, {96, 128}), ("s2", 8.0, {32}), ("s2", 40.0, {64}), ("s2", 60.0, {64, 96})])
+def test_small_sets(key, weak, sizes, mode, oracle_mod, monkeypatch):
     import ecp_cases
     from ctemsoft_amd import ebsd, ecp
     z = fixture()
@@ -38,6 +38,7 @@ def test_small_sets(key, weak, mode, oracle_mod, monkeypatch):
     finally:
         ctx.close()
     assert np.isfinite(sr).all()
+    assert set(((ns + 31) // 32 * 32).tolist()) == sizes
     order = np.argsort(ns, kind="stable")
     pick = np.unique(np.concatenate([order[[0, 1, -2, -1]], order[::max(1, len(order) // 8)]]))
     print(f"{key} {weak} {mode}: {ns.min()}..{ns.max()} beams, {len(pick)} directions", flush=True)
