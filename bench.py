@@ -523,7 +523,7 @@ def bench_ecp(a):
                      "frac": None if ach is None else round(ach / 78.6, 4), "traffic": None,
                      "kernel": "k_ecp_bloch_small" if small else "k_zgemm, k_ecp_bloch_small up to 64 beams",
                      "alg_flops_per_step": b["gemm_flops"], "kernel_ms_per_step": round(b["gemm_ms"], 3),
-                     "kernel_ms_source": "HIP events around those launches on the context's stream",
+                     "kernel_ms_source": "the device's wall clock in k_ecp_bloch_small, HIP events around k_zgemm",
                      "note": "FP64 complex products on the true sizes: up to 64 strong beams (n) the exponential and the doubled "
                              "thickness integral, 8 n^3 flops each, in one kernel with everything after the dynamical matrix; "
                              "past that the block-matrix exponentials, 8 (2n)^3"},

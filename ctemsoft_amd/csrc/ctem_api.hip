@@ -230,7 +230,7 @@ struct ctem_plan {
   // electron channeling pattern plan (ctem_ecp_plan_create): mode, thicknesses, the foil normal
   // of the selection, the channeling structure matrix table, ScatMat's store map and the results
   int32_t ecp_mode = -1;  // -1: a master-pattern plan
-  int32_t ecp_nt = 0, ecp_numt = 0;
+  int32_t ecp_nt = 0, ecp_numt = 0, ecp_clocks = 0;
   float ecp_t0 = 0.0f, ecp_dt = 0.0f, ecp_zint = 0.0f;
   double ecp_nat = 1.0, ecp_s0 = 1.0;
   DBuf selbits;  // the beam selection's class masks
@@ -2092,25 +2092,33 @@ extern "C" int32_t ctem_plan_scatter(ctem_plan* p, const int32_t* ij, int32_t np
   return CTEM_OK;
 }
 
-// The products of a channeling plan's one-launch directions, kept behind its intensities: int32 per direction, 0 for others
-static size_t ecp_nprod_at(const ctem_plan* p) { return sizeof(float) * (size_t)p->ecp_nt * std::max(p->numk, 1); }
+// Behind a channeling plan's intensities: the clocks of up to kEcpClocks one-launch chunks (later ones share the last)
+// and the products of their directions (EcpStat)
+constexpr int kEcpClocks = 64;
+static size_t ecp_stat_at(const ctem_plan* p) {
+  return (sizeof(float) * (size_t)p->ecp_nt * std::max(p->numk, 1) + 7) / 8 * 8;
+}
+static size_t ecp_stat_bytes(const ctem_plan* p) { return 16 * kEcpClocks + 4 * (size_t)std::max(p->numk, 1); }
 
 extern "C" int32_t ctem_plan_timing(ctem_plan* p, double* total_ms, double* gemm_ms, double* gemm_flops,
                                     int32_t* gemm_launches) {
   if (!p || !p->ran) return fail(CTEM_E_STATE, "ctem_plan_timing: run the plan first");
   if (total_ms) *total_ms = p->t_total;
-  if (gemm_ms) *gemm_ms = p->t_gemm;
-  if (gemm_flops) {
-    double f = 0.0;
-    if (p->ecp_mode >= 0 && p->numk > 0) {
-      std::vector<int32_t> np(p->numk);
-      HIPCHK(hipMemcpy(np.data(), (char*)p->ecp_sr.p + ecp_nprod_at(p), 4 * np.size(), hipMemcpyDeviceToHost));
-      const double solve = p->ecp_mode == CTEM_ECP_SCATMAT ? 32.0 / 3.0 : 0.0;
-      for (int i = 0; i < p->numk; i++)
-        if (np[i]) f += (double)p->h_nns[i] * p->h_nns[i] * p->h_nns[i] * (8.0 * np[i] + solve);
-    }
-    *gemm_flops = p->f_gemm + f;
+  double ms = 0.0, f = 0.0;
+  if (p->ecp_mode >= 0 && p->ecp_clocks > 0) {
+    std::vector<char> buf(ecp_stat_bytes(p));
+    HIPCHK(hipMemcpy(buf.data(), (char*)p->ecp_sr.p + ecp_stat_at(p), buf.size(), hipMemcpyDeviceToHost));
+    const auto* clk = (const unsigned long long*)buf.data();
+    const auto* np = (const int32_t*)(buf.data() + 16 * kEcpClocks);
+    int khz = 0;
+    HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, p->ctx->device));
+    for (int i = 0; i < p->ecp_clocks; i++) ms += (double)(clk[2 * i + 1] - ~clk[2 * i]) / khz;
+    const double solve = p->ecp_mode == CTEM_ECP_SCATMAT ? 32.0 / 3.0 : 0.0;
+    for (int i = 0; i < p->numk; i++)
+      if (np[i]) f += (double)p->h_nns[i] * p->h_nns[i] * p->h_nns[i] * (8.0 * np[i] + solve);
   }
+  if (gemm_ms) *gemm_ms = p->t_gemm + ms;
+  if (gemm_flops) *gemm_flops = p->f_gemm + f;
   if (gemm_launches) *gemm_launches = p->n_gemm;
   return CTEM_OK;
 }
@@ -2461,7 +2469,7 @@ extern "C" int32_t ctem_ecp_plan_create(ctem_ctx* c, int32_t numk, const double*
   if ((rc = upload(p->fn, prm->fn, 3, s)) || (rc = upload(p->ecp_slut, slut.data(), slut.size(), s)) ||
       (rc = upload(p->ecp_thick, thick.data(), thick.size(), s)) ||
       (numt > 0 && (rc = upload(p->ecp_store, store.data(), store.size(), s))) ||
-      (rc = p->ecp_sr.ensure(ecp_nprod_at(p) + 4 * (size_t)std::max(numk, 1)))) {
+      (rc = p->ecp_sr.ensure(ecp_stat_at(p) + ecp_stat_bytes(p)))) {
     ctem_plan_destroy(p);
     *out = nullptr;
     return rc;
@@ -2527,8 +2535,9 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
   reset_timing(p);
   HIPCHK(hipEventRecord(c->ev[0], s));
   launch_fill_zero(s, p->err.p, 4);
-  launch_fill_zero(s, p->ecp_sr.p, ecp_nprod_at(p) + 4 * (size_t)std::max(p->numk, 1));
-  int32_t* nprod = (int32_t*)((char*)p->ecp_sr.p + ecp_nprod_at(p));
+  launch_fill_zero(s, p->ecp_sr.p, ecp_stat_at(p) + ecp_stat_bytes(p));
+  auto* clocks = (unsigned long long*)((char*)p->ecp_sr.p + ecp_stat_at(p));
+  p->ecp_clocks = 0;
   BeamView V{p->nns.as<int32_t>(), p->nnw.as<int32_t>(), p->soff.as<int64_t>(), p->woff.as<int64_t>(),
              p->sidx.as<int32_t>(), p->ssg.as<float>(), p->widx.as<int32_t>(), p->wsg.as<float>()};
   DevRefl R = p->cr->refl();
@@ -2550,15 +2559,14 @@ extern "C" int32_t ctem_ecp_run(ctem_plan* p) {
         double2* A = c->w.A.as<double2>();
         if (bloch) launch_assemble(s, B, V, R, L, p->kn.as<double>(), p->cr->mlambda, p->cr->dynupz, 1.0, A);
         else launch_assemble_scatmat(s, B, V, R, L, p->cr->mlambda, p->cr->dynupz, (double)p->ecp_zint, A);
-        GemmTimer t{p, s};
-        t.begin();
+        const EcpStat stat{clocks + 2 * std::min(p->ecp_clocks, kEcpClocks - 1), (int32_t*)(clocks + 2 * kEcpClocks)};
         if (bloch)
           launch_ecp_bloch_small(s, B, V, R, LE, A, (double)p->ecp_t0, (double)p->ecp_dt, nt, p->ecp_thick.as<float>(),
-                                 p->ecp_nat, p->numk, p->err.as<int32_t>(), p->ecp_sr.as<float>(), nprod);
+                                 p->ecp_nat, p->numk, p->err.as<int32_t>(), p->ecp_sr.as<float>(), stat);
         else
           launch_ecp_scat_small(s, B, V, R, LE, A, numt, p->ecp_store.as<int32_t>(), p->ecp_nat, p->numk,
-                                p->err.as<int32_t>(), p->ecp_sr.as<float>(), nprod);
-        t.end();
+                                p->err.as<int32_t>(), p->ecp_sr.as<float>(), stat);
+        p->ecp_clocks = std::min(p->ecp_clocks + 1, kEcpClocks);
         p->n_gemm++;
         HIPCHK(hipGetLastError());
       } else if (!bloch) {

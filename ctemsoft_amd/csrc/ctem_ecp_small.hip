@@ -138,6 +138,15 @@ __device__ __forceinline__ double2 sgh_at(const DevRefl& R, const DevLut& L, int
                 (int64_t)L.sdim[0] * ((x[1] - y[1] - L.slo[1]) + (int64_t)L.sdim[1] * (x[2] - y[2] - L.slo[2]))];
 }
 
+// The launch's time, from its first workgroups' start to its last ones' end, without events around it (those cost
+// 10 us a launch, of 60-150 for a hundred directions)
+__device__ __forceinline__ void stat_begin(const EcpStat& s) {
+  if (threadIdx.x == 0 && blockIdx.x < 64) atomicMax(s.clock, ~(unsigned long long)wall_clock64());
+}
+__device__ __forceinline__ void stat_end(const EcpStat& s) {
+  if (threadIdx.x == 0 && blockIdx.x + 2048 >= gridDim.x) atomicMax(s.clock + 1, (unsigned long long)wall_clock64());
+}
+
 // Taylor at ||A h|| <= 1/8 (1-norms of A h and its conjugate transpose): E to degree 12 (five products), M to
 // the term of degree 11 in the map X -> X A + (X A)^H (a product each); the first terms left out are
 // below 1e-21 and 1e-17. A larger bound saves three products per doubling and costs as many here
@@ -148,7 +157,7 @@ template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4 : 1, NT == 1 ? 4 : 1)))
 void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* __restrict__ A1, double t0, double dt,
                        int nt, const float* __restrict__ thick, double nat, int numk, int32_t* __restrict__ err,
-                       float* __restrict__ sr, int32_t* __restrict__ nprod) {
+                       float* __restrict__ sr, EcpStat stat) {
   typedef Wg<NT> W;
   constexpr int NP = W::NP, LD = W::LD;
   extern __shared__ double2 lds[];
@@ -157,6 +166,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
   double2* const psi = P1 + NP * LD;
   double* const red = (double*)(psi + 2 * NP);
   const int b = blockIdx.x, dir = B.dirs[b], n = V.nns[dir], tid = threadIdx.x;
+  stat_begin(stat);
   const W w(n);
   const int32_t* sidx = V.sidx + V.soff[dir];
   const double2* A = A1 + (int64_t)b * NP * NP;
@@ -279,8 +289,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
   if (tid < NP) psi[tid] = P0[tid];
   if (tid == 0) sr[dir] = (float)(run / (double)thick[0] / nat);
   if (nt >= 2 && dt != t0) propagators(dt);
-  if (tid == 0) nprod[dir] = products;
-  if (nt < 2) return;
+  if (tid == 0) stat.nprod[dir] = products;
   __syncthreads();
   for (int it = 1; it < nt; it++) {
     const double2* u = psi + ((it - 1) & 1) * NP;
@@ -297,13 +306,14 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
       sr[(int64_t)it * numk + dir] = (float)(run / (double)thick[it] / nat);
     }
   }
+  stat_end(stat);
 }
 
 template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NT == 1 ? 4 : 1)))
 void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* __restrict__ A1, int nz,
                       const int32_t* __restrict__ store, double nat, int numk, int32_t* __restrict__ err,
-                      float* __restrict__ sr, int32_t* __restrict__ nprod) {
+                      float* __restrict__ sr, EcpStat stat) {
   typedef Wg<NT> W;
   constexpr int NP = W::NP, LD = W::LD;
   extern __shared__ double2 lds[];
@@ -312,6 +322,7 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
   double2* const psi = P1 + NP * LD;
   double* const red = (double*)(psi + 2 * NP);
   const int b = blockIdx.x, dir = B.dirs[b], n = V.nns[dir], tid = threadIdx.x;
+  stat_begin(stat);
   const W w(n);
   const int32_t* sidx = V.sidx + V.soff[dir];
   const double2* A = A1 + (int64_t)b * NP * NP;
@@ -335,7 +346,7 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
   const int q = ilev == 1 ? 2 : ilev == 2 ? 3 : 4;
   const int j2 = ilev <= 2 ? 0 : ilev == 3 ? 1 : ilev == 4 ? 5 : ilev == 5 ? 8 : 11;
   const double sc = ldexp(1.0, -j2);
-  if (tid == 0) nprod[dir] = q - 1 + j2;
+  if (tid == 0) stat.nprod[dir] = q - 1 + j2;
   // N = sum pref_i B^i, D = sum (-1)^i pref_i B^i with the reference's running product pref
   w.each([&](int i, int j, int e, int r, int c) {
     double2 v = P0[c * LD + r];
@@ -478,6 +489,7 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
       sr[(int64_t)t * numk + dir] = (float)(((q[0] + q[1]) + (q[2] + q[3])) / nat);
     }
   }
+  stat_end(stat);
 }
 
 }  // namespace
@@ -487,24 +499,24 @@ bool ecp_small(int npad) { return npad <= 64; }
 
 void launch_ecp_bloch_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                             const double2* A1, double t0, double dt, int32_t nt, const float* thick, double nat,
-                            int32_t numk, int32_t* err, float* sr, int32_t* nprod) {
+                            int32_t numk, int32_t* err, float* sr, const EcpStat& stat) {
   if (B.npad == 32)
     hipLaunchKernelGGL(k_ecp_bloch_small<1>, dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
-                       nat, numk, err, sr, nprod);
+                       nat, numk, err, sr, stat);
   else
     hipLaunchKernelGGL(k_ecp_bloch_small<2>, dim3(B.nb), dim3(256), Wg<2>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
-                       nat, numk, err, sr, nprod);
+                       nat, numk, err, sr, stat);
 }
 
 void launch_ecp_scat_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                            const double2* A1, int32_t nz, const int32_t* store, double nat, int32_t numk, int32_t* err,
-                           float* sr, int32_t* nprod) {
+                           float* sr, const EcpStat& stat) {
   if (B.npad == 32)
     hipLaunchKernelGGL(k_ecp_scat_small<1>, dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, nz, store, nat, numk,
-                       err, sr, nprod);
+                       err, sr, stat);
   else
     hipLaunchKernelGGL(k_ecp_scat_small<2>, dim3(B.nb), dim3(256), Wg<2>::lds(), s, B, V, R, L, A1, nz, store, nat, numk,
-                       err, sr, nprod);
+                       err, sr, stat);
 }
 
 }  // namespace ctem

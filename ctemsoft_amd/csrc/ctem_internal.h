@@ -376,15 +376,18 @@ void launch_ecp_bloch_steps(hipStream_t s, const Bucket& B, const BeamView& V, c
                             const float* thick, double eps, double nat, int32_t numk, float* sr);
 
 // up to 64 strong beams (ecp_small(npad)): everything after the dynamical matrix in one launch
-// (ctem_ecp_small.hip); err receives 2 for a non-finite matrix or a zero pivot, 4 for a norm out of range; nprod[direction]
-// the matrix products taken
+// (ctem_ecp_small.hip); err receives 2 for a non-finite matrix or a zero pivot, 4 for a norm out of range
 bool ecp_small(int npad);
+struct EcpStat {
+  unsigned long long* clock;  // of the launch, zeroed: ~start and end in ticks of the device's wall clock
+  int32_t* nprod;             // [direction] matrix products taken
+};
 void launch_ecp_bloch_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                             const double2* A1, double t0, double dt, int32_t nt, const float* thick, double nat,
-                            int32_t numk, int32_t* err, float* sr, int32_t* nprod);
+                            int32_t numk, int32_t* err, float* sr, const EcpStat& stat);
 void launch_ecp_scat_small(hipStream_t s, const Bucket& B, const BeamView& V, const DevRefl& R, const DevLut& L,
                            const double2* A1, int32_t nz, const int32_t* store, double nat, int32_t numk, int32_t* err,
-                           float* sr, int32_t* nprod);
+                           float* sr, const EcpStat& stat);
 
 // MatrixExponential 'Pade' (math.f90:187-315), batched over nb npad x npad matrices A (holding
 // A z0): prep scales A to B = A / 2^j in place and sets N = D = I, C = B, qm1[b] = q - 1, jj[b] = j;

@@ -204,7 +204,8 @@ CTEM_API int32_t ctem_plan_scatter(ctem_plan* plan, const int32_t* ij, int32_t n
 /* Timing of the last ctem_plan_run, measured with HIP events on the context's stream:
  * total milliseconds and milliseconds in the dominant (matrix-exponential GEMM) kernels,
  * with the algorithmic flop count of those kernels. Of a channeling-pattern plan's ctem_ecp_run, directions
- * of up to 64 strong beams count with everything after the dynamical matrix (one kernel). */
+ * of up to 64 strong beams count with everything after the dynamical matrix (one kernel, timed by the
+ * device's wall clock). */
 CTEM_API int32_t ctem_plan_timing(ctem_plan* plan, double* total_ms, double* gemm_ms, double* gemm_flops,
                          int32_t* gemm_launches);
 
