@@ -32,7 +32,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // FN = k of each direction. One workgroup per direction, 64 reflections per wave and step, no barriers in the
 // loop. The counting pass (fill = 0) leaves each wave's two class masks in out.bits; the filling pass computes s_g
 // only for the beams that are set there. Bound by the program's acosf/cosf arithmetic of the counting pass.
-// bcc Fe, 21,000 directions: both passes 1.34 -> 0.77 ms against computing s_g twice with three barriers a step.
+// bcc Fe, 63,252 directions: both passes 1.34 -> 0.78 ms against computing s_g twice with three barriers a step.
 template <bool FILL>
 __global__ __launch_bounds__(256) void k_select(const double* __restrict__ kvec, int32_t numk,
                                                 DevRefl R, const double* __restrict__ rmt_g,
@@ -373,13 +373,13 @@ void launch_norm_scale(hipStream_t s, int32_t npad, int32_t nb, double2* A, doub
 // four consecutive rows). Y is passed as A and X as B, so that 16 lanes hold 16 consecutive rows of C.
 //
 // k_zgemm: workgroup tile 64x64, 4 waves of 32x32, K in chunks of 8 that the load unit writes to LDS (two
-// buffers, one barrier a chunk). Bound by the matrix cores: 64 MFMAs of 64 cycles per SIMD and chunk
+// buffers, one barrier a chunk). Bound by the matrix cores: 32 MFMAs of 64 cycles per SIMD and chunk
 // against 16 KB staged. A matrix's own size n (its beams, of npad) cuts K to multiples of 8 and the waves'
 // tiles to multiples of 16; the zero padding past it is written, not multiplied. The waves' places in the
 // tile turn with the matrix, so that the waves with cut tiles are spread over the four SIMDs. 110 registers,
 // four workgroups per CU (three are 15% slower). Measured on one MI355X against chunks staged through registers
 // with the accumulators moved each chunk: the products of 1,326 matrices of 87-115 beams and their adjoint
-// pairs 26.0 -> 16.8 ms, half of it matrix-core time, with 40 GB of operands moved; bcc Fe FP64 master of
+// pairs 26.0 -> 16.5 ms, with the matrix cores 57% busy and 56 GB of operands moved; bcc Fe FP64 master of
 // up to 224 beams 34.4 -> 26 ms.
 constexpr int kZgemmFew = 256;  // 64x64 tiles: one per CU
 struct ZgOperands {  // of one result: np products of X[p] and Y[p]
@@ -862,7 +862,7 @@ __global__ __launch_bounds__(1024) void k_depth_onchip(int nb, int nz, const flo
 // The same recursion for up to 32 beams (FP32 storage): one wave per matrix and no barriers. Lane (r, h) holds
 // columns 16 h .. 16 h + 15 of row r in registers, the halves of a row meet by a lane swap, and the FP32 copy of
 // the vector goes through the wave's own 256 bytes of LDS. Bound by the vector unit (64 multiply-adds a step);
-// one MI355X, bcc Fe of 5-27 beams, 50 depths: the master pattern's launch 5.03 -> 0.40 ms against a 1024-thread
+// one MI355X, bcc Fe of 1-14 beams, 63,252 directions, 50 depths: the master pattern's launch 5.03 -> 0.40 ms against a 1024-thread
 // workgroup per matrix with a barrier a step. (64 beams would take 128 registers for the rows alone.)
 __global__ __launch_bounds__(256) void k_depth_wave(int nb, int nz, const float2* __restrict__ E, int add_identity,
                                                     double2* __restrict__ Psi, int64_t spsi) {

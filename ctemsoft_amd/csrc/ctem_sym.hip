@@ -24,7 +24,7 @@
 //
 // Measured on one MI355X, the exponentials of a run against k_sgemm's chain (64 x 64 tiles, three general
 // products for a degree-8 polynomial; it moves 2.3 MB to LDS per product at n = 224 and waits for memory):
-// bcc Fe, 63,252 directions of 188-250 beams: 142 -> 87 ms, with 9-10 products per matrix instead of 8; fcc Ni, 1,326 of
+// bcc Fe, 63,252 directions of 188-250 beams: 142 -> 87 ms, with 9 products per matrix instead of 8; fcc Ni, 1,326 of
 // 87-115: 1.03 -> 0.48 ms. Intensities against 64 bits over 140 drawn sets: the 2-norm error is 0.57-0.72 of that chain's
 // on average at every size, at most 1.13 of it.
 #include <hip/hip_runtime.h>
