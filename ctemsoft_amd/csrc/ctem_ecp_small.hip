@@ -11,13 +11,14 @@
 //   k_ecp_scat_small    ScatMat: the program's Pade approximant (math.f90:187-315), the depth recursion
 //                       and the per-depth contraction with S (CTEMECP.f90:559-618)
 //
-// 256 threads; products on v_mfma_f64_16x16x4_f64, each wave one quadrant of the matrix. LDS matrices
-// are column-major with one spare row, which keeps both operands' reads free of bank conflicts.
+// 256 threads (1024 in Blochwv past 32 beams); products on v_mfma_f64_16x16x4_f64, each wave one part of the matrix. LDS
+// matrices are column-major with one spare row, which keeps both operands' reads free of bank conflicts.
 // Bound: FP64 matrix cores in Blochwv; in ScatMat half the time is the elimination, on the FP64 vector unit.
-// Four workgroups per CU at 32 beams (35 KB of LDS, 128 registers), one at 64. One MI355X, fcc Ni [001] at 30 kV,
+// Four workgroups per CU at 32 beams (35 KB of LDS, 128 registers), one at 64: with four waves there a single direction of
+// 45 beams at 200-650 nm took 940 us, more than the batched form's 876, with sixteen 801. One MI355X, fcc Ni [001] at 30 kV,
 // 16-32 beams, a pass against the batched form: Blochwv, 12,853 directions and 10 thicknesses, 19.9 -> 2.2 ms;
-// ScatMat, 51,400 directions and 20 steps, 25.6 -> 5.2 ms. 40-57 beams (15 kV), 1,793 directions: Blochwv 17.6 -> 5.9,
-// ScatMat 5.3 -> 1.6 ms. At 96 two matrices don't fit in LDS.
+// ScatMat, 51,400 directions and 20 steps, 25.6 -> 5.2 ms. 40-57 beams (15 kV), 1,256 directions: Blochwv 12.7 -> 2.0,
+// ScatMat 3.5 -> 1.2 ms. At 96 two matrices don't fit in LDS.
 #include <hip/hip_runtime.h>
 
 #include "ctem_ebsd.h"
@@ -44,38 +45,42 @@ __device__ __forceinline__ double lane_of(double v, int l) {  // lane l's v, in 
   return __longlong_as_double(((uint64_t)hi << 32) | lo);
 }
 
-// max over the workgroup, the same in every thread (a NaN wins); red: four doubles of LDS
+// max over the workgroup of NW waves, the same in every thread (a NaN wins); red: NW doubles of LDS
+template <int NW>
 __device__ __forceinline__ double block_max(double v, double* red) {
   auto mx = [](double a, double b) { return (a != a) ? a : ((b != b) ? b : fmax(a, b)); };
   for (int o = 32; o >= 1; o >>= 1) v = mx(v, __shfl_xor(v, o, 64));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  return mx(mx(red[0], red[1]), mx(red[2], red[3]));
+  v = red[0];
+#pragma unroll
+  for (int w = 1; w < NW; w++) v = mx(v, red[w]);
+  return v;
 }
 
-// The workgroup's view of NP x NP matrices (NP = 32 NT): thread-owned entries (i, j, e) are row
-// row(i, e), column col(j) of the wave's quadrant, the accumulator layout of the products.
-template <int NT>
+// The workgroup's view of NP x NP matrices (NP = 32 NT; four waves, each a quadrant, or sixteen): thread-owned
+// entries (i, j, e) are row row(i, e), column col(j) of the wave's part, the accumulator layout of the products.
+template <int NT, int NW = 4>
 struct Wg {
-  static constexpr int NP = 32 * NT, LD = NP + 1, NE = 4 * NT * NT;
-  typedef d4 Acc[NT][NT];
+  static constexpr int NP = 32 * NT, LD = NP + 1, WS = NW == 16 ? 4 : 2, TW = 2 * NT / WS, NTH = 64 * NW;
+  typedef d4 Acc[TW][TW];
   int l16, l4, wr, wc, n, kn;
   // n: the matrix's own size; rows and columns from there on are those of the zero or the unit matrix,
   // and no sum over k goes past kn
   __device__ __forceinline__ explicit Wg(int n_) : n(n_), kn((n_ + 7) & ~7) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     l16 = lane & 15; l4 = lane >> 4;
-    wr = (wave >> 1) * 16 * NT; wc = (wave & 1) * 16 * NT;
+    wr = (wave / WS) * 16 * TW; wc = (wave % WS) * 16 * TW;
   }
   __device__ __forceinline__ int row(int i, int e) const { return wr + 16 * i + l4 + 4 * e; }
   __device__ __forceinline__ int col(int j) const { return wc + 16 * j + l16; }
   template <class F>
   __device__ __forceinline__ void each(F f) const {
 #pragma unroll
-    for (int i = 0; i < NT; i++)
+    for (int i = 0; i < TW; i++)
 #pragma unroll
-      for (int j = 0; j < NT; j++)
+      for (int j = 0; j < TW; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) f(i, j, e, row(i, e), col(j));
   }
@@ -83,24 +88,24 @@ struct Wg {
   template <bool HERM>
   __device__ __forceinline__ void mul(const double2* X, const double2* Y, Acc& cr, Acc& ci) const {
 #pragma unroll
-    for (int i = 0; i < NT; i++)
+    for (int i = 0; i < TW; i++)
 #pragma unroll
-      for (int j = 0; j < NT; j++) { cr[i][j] = (d4){0, 0, 0, 0}; ci[i][j] = (d4){0, 0, 0, 0}; }
+      for (int j = 0; j < TW; j++) { cr[i][j] = (d4){0, 0, 0, 0}; ci[i][j] = (d4){0, 0, 0, 0}; }
     for (int k0 = 0; k0 < kn; k0 += 8)
 #pragma unroll
     for (int k = k0; k < k0 + 8; k += 4) {
-      double2 a[NT], b[NT];
+      double2 a[TW], b[TW];
 #pragma unroll
-      for (int i = 0; i < NT; i++) {
+      for (int i = 0; i < TW; i++) {
         const int r = wr + 16 * i + l16;
         a[i] = HERM ? X[r * LD + k + l4] : X[(k + l4) * LD + r];
         if (HERM) a[i].y = -a[i].y;
         b[i] = Y[(wc + 16 * i + l16) * LD + k + l4];
       }
 #pragma unroll
-      for (int i = 0; i < NT; i++)
+      for (int i = 0; i < TW; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
+        for (int j = 0; j < TW; j++) {
           cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, cr[i][j], 0, 0, 0);
           ci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].y, ci[i][j], 0, 0, 0);
           cr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[i].y, b[j].y, cr[i][j], 0, 0, 0);
@@ -113,7 +118,7 @@ struct Wg {
   }
   // x = X u, the sum of row tid / G in each of its G threads; y = this thread's part of row tid / G of
   // Y u (or Y conj(u))
-  static constexpr int G = 256 / NP;
+  static constexpr int G = NTH / NP;
   template <bool CONJ>
   __device__ __forceinline__ void matvec2(const double2* X, const double2* Y, const double2* u, double2& x, double2& y) const {
     const int r = threadIdx.x / G, g = threadIdx.x % G;
@@ -126,7 +131,8 @@ struct Wg {
     }
     x.x += dpp_f64<0xb1>(x.x); x.y += dpp_f64<0xb1>(x.y);  // quad_perm [1,0,3,2]
     x.x += dpp_f64<0x4e>(x.x); x.y += dpp_f64<0x4e>(x.y);  // quad_perm [2,3,0,1]
-    if (G == 8) { x.x += dpp_f64<0x141>(x.x); x.y += dpp_f64<0x141>(x.y); }  // row_half_mirror
+    if (G >= 8) { x.x += dpp_f64<0x141>(x.x); x.y += dpp_f64<0x141>(x.y); }  // row_half_mirror
+    if (G == 16) { x.x += dpp_f64<0x140>(x.x); x.y += dpp_f64<0x140>(x.y); }  // row_mirror
   }
   static constexpr size_t lds() { return (size_t)(2 * NP * LD + 2 * NP) * sizeof(double2) + 64 * sizeof(double); }
 };
@@ -153,12 +159,12 @@ __device__ __forceinline__ void stat_end(const EcpStat& s) {
 constexpr double kThetaSmall = 0.125;
 constexpr int kDegM = 11, kSmaxSmall = 51;  // 2^51 kThetaSmall is beyond the range of the larger sets' 48 squarings
 
-template <int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4 : 1, NT == 1 ? 4 : 1)))
+template <int NT, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* __restrict__ A1, double t0, double dt,
                        int nt, const float* __restrict__ thick, double nat, int numk, int32_t* __restrict__ err,
                        float* __restrict__ sr, EcpStat stat) {
-  typedef Wg<NT> W;
+  typedef Wg<NT, NW> W;
   constexpr int NP = W::NP, LD = W::LD;
   extern __shared__ double2 lds[];
   double2* const P0 = lds;
@@ -171,7 +177,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
   const int32_t* sidx = V.sidx + V.soff[dir];
   const double2* A = A1 + (int64_t)b * NP * NP;
   // the norms of A
-  for (int e = tid; e < NP * NP; e += 256) P0[(e / NP) * LD + e % NP] = A[e];
+  for (int e = tid; e < NP * NP; e += W::NTH) P0[(e / NP) * LD + e % NP] = A[e];
   __syncthreads();
   double nrm = 0.0;
   if (tid < 2 * NP) {
@@ -181,8 +187,8 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
       nrm += hypot(v.x, v.y);
     }
   }
-  nrm = block_max(nrm, red);
-  double2 sp[NT][NT][4];  // S^T: Sgh(hkl_c - hkl_r)
+  nrm = block_max<NW>(nrm, red);
+  double2 sp[W::TW][W::TW][4];  // S^T: Sgh(hkl_c - hkl_r)
   w.each([&](int i, int j, int e, int r, int c) {
     sp[i][j][e] = (r < n && c < n) ? sgh_at(R, L, sidx[c], sidx[r]) : make_double2(0.0, 0.0);
   });
@@ -202,7 +208,7 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
     products += kDegM + 5 + 3 * s;
     typename W::Acc er, ei, mr, mi, cr, ci;
     __syncthreads();
-    for (int e = tid; e < NP * NP; e += 256) {
+    for (int e = tid; e < NP * NP; e += W::NTH) {
       const double2 v = A[e];
       P0[(e / NP) * LD + e % NP] = make_double2(v.x * h, v.y * h);
     }
@@ -298,11 +304,12 @@ void k_ecp_bloch_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2*
     const int r = tid / W::G;
     if (tid % W::G == 0) psi[(it & 1) * NP + r] = x;
     const double v = wave_sum(u[r].x * y.x + u[r].y * y.y);
-    if ((tid & 63) == 0) red[4 * (it & 1) + (tid >> 6)] = v;
+    if ((tid & 63) == 0) red[NW * (it & 1) + (tid >> 6)] = v;
     __syncthreads();
     if (tid == 0) {
-      const double* q = red + 4 * (it & 1);
-      run += (q[0] + q[1]) + (q[2] + q[3]);
+      const double* q = red + NW * (it & 1);
+#pragma unroll
+      for (int g = 0; g < NW; g += 4) run += (q[g] + q[g + 1]) + (q[g + 2] + q[g + 3]);
       sr[(int64_t)it * numk + dir] = (float)(run / (double)thick[it] / nat);
     }
   }
@@ -335,7 +342,7 @@ void k_ecp_scat_small(Bucket B, BeamView V, DevRefl R, DevLut L, const double2* 
     m = (a > m || a != a) ? a : m;
     P0[(e / NP) * LD + e % NP] = v;
   }
-  m = block_max(m, red);
+  m = block_max<4>(m, red);
   int ilev = 1;
   if (!(m == m) || m > 1000.0) {
     if (tid == 0) atomicOr(err, 4);
@@ -501,10 +508,10 @@ void launch_ecp_bloch_small(hipStream_t s, const Bucket& B, const BeamView& V, c
                             const double2* A1, double t0, double dt, int32_t nt, const float* thick, double nat,
                             int32_t numk, int32_t* err, float* sr, const EcpStat& stat) {
   if (B.npad == 32)
-    hipLaunchKernelGGL(k_ecp_bloch_small<1>, dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
+    hipLaunchKernelGGL((k_ecp_bloch_small<1, 4>), dim3(B.nb), dim3(256), Wg<1>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
                        nat, numk, err, sr, stat);
   else
-    hipLaunchKernelGGL(k_ecp_bloch_small<2>, dim3(B.nb), dim3(256), Wg<2>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
+    hipLaunchKernelGGL((k_ecp_bloch_small<2, 16>), dim3(B.nb), dim3(1024), Wg<2>::lds(), s, B, V, R, L, A1, t0, dt, nt, thick,
                        nat, numk, err, sr, stat);
 }
 
