@@ -1116,7 +1116,8 @@ int32_t expm_depth_mixed(ctem_plan* tp, hipStream_t s, int npad, int nb, float2*
 
 // The complex-symmetric form of expm_depth_split, for the sizes that sym_onchip accepts. Buffers (8 bytes
 // per entry): 0 A as assembled, 1 B^2, 2 the tile images that do not fit on chip, 3 the FP32 F for the
-// depth kernel. wmax holds maxima and exponents as in expm_depth_split.
+// depth kernel; a few matrices (sym_few): 1 B, 2 B^2, 4 and 5 the operands. wmax holds maxima and exponents as in
+// expm_depth_split.
 int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
                        const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz, int32_t* d_sq,
                        int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq, int depth_grid,
@@ -1170,7 +1171,8 @@ int32_t expm_depth_sym(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W
 // Taylor products as B = A 2^-s (split on the fly when staged); 1 L; 2 B2; 3 P, later the FP32
 // copy of the final F of every matrix (written by its last product) for the depth kernel; 4 R,
 // then the squarings alternate between 5 (F0) and 4. wmax holds six FP32 maxima and six
-// exponents per matrix (slot 0: L, slot 1: B, slots 2-5 as the buffers), then the max of A.
+// exponents per matrix (slot 0: L, slot 1: B, slots 2-5 as the buffers), then the max of A. Symmetric matrices
+// of up to 224 beams go to expm_depth_sym with `squares`.
 int32_t expm_depth_split(ctem_plan* tp, hipStream_t s, int npad, int nb, float2* W32, const double* colpart,
                          const float* amax, float* wmax, double2* Psi64, int64_t spsi, int nz,
                          int32_t* d_sq, int32_t* d_err, const std::vector<int>& h_n, std::vector<int32_t>& h_sq,
